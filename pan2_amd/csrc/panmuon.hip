@@ -16,6 +16,7 @@
 #include "../../include/panmuon.h"
 #include "pm_kernels.hpp"
 #include "pm_small.hpp"
+#include "pm_mid.hpp"
 #include "pm_adam.hpp"
 
 using namespace pm;
@@ -411,6 +412,8 @@ struct Launcher {
     const int32_t* items;   // split matrices' work items (tiles x chunks)
     const int32_t* split;   // split matrices' tiles
     int32_t tiles_total, items_total, split_total;
+    int edge;               // tile edge: kTile, or the small-tile engine's 128 or 64
+    bool persistent;        // small-tile engine: one block per CU
   };
   Stage gram_s, sym_s, full_s;
   int32_t* queues;      // kXcds counters per GEMM launch, zero at upload
@@ -429,8 +432,32 @@ struct Launcher {
   // when some matrix splits this stage, the GEMM over their chunk items
   // (fp32 partials) and the reduce over their tiles. The stage's FLOPs go
   // with its first launch.
+  template <int STAGE, int T, int NW, int RING>
+  int tile_launch(GemmArgs a, const Stage& st, int kind, int it, double flops, const char* what) {
+    if (st.tiles_total > 0) {
+      a.prefix = st.tiles;
+      a.total = st.tiles_total;
+      hipLaunchKernelGGL((pm_tile_gemm_kernel<STAGE, T, NW, RING, false>), dim3(st.persistent ? gemm_grid(a.total) : a.total), dim3(64 * NW), 0, stream, a);
+      timing_mark(stream, kind, group, it, count, flops, 0.0);
+      flops = 0.0;
+      if (int rc = check(what)) return rc;
+    }
+    if (st.items_total == 0) return PM_OK;
+    a.prefix = st.items;
+    a.total = st.items_total;
+    hipLaunchKernelGGL((pm_tile_gemm_kernel<STAGE, T, NW, RING, true>), dim3(st.persistent ? gemm_grid(a.total) : a.total), dim3(64 * NW), 0, stream, a);
+    timing_mark(stream, kind, group, it, count, flops, 0.0);
+    if (int rc = check(what)) return rc;
+    a.prefix = st.split;
+    a.total = st.split_total;
+    hipLaunchKernelGGL((pm_tile_reduce_kernel<STAGE, T, NW>), dim3(a.total), dim3(64 * NW), 0, stream, a);
+    timing_mark(stream, PM_K_REDUCE, group, it, count, 0.0, 0.0);
+    return check("K-split reduce launch");
+  }
   template <int STAGE, int PDT>
   int stage_launch(GemmArgs a, const Stage& st, int kind, int it, double flops, const char* what) {
+    if (st.edge == 64) return tile_launch<STAGE, 64, 4, 4>(a, st, kind, it, flops, what);
+    if (st.edge == 128) return tile_launch<STAGE, 128, 8, 4>(a, st, kind, it, flops, what);
     if (st.tiles_total > 0) {
       a.prefix = st.tiles;
       a.total = st.tiles_total;
@@ -630,6 +657,65 @@ int run_small(Launcher& L, const pm_hparams* hp, bool fused, bool pro_gram) {
 // (load_table_by_kernel: no staging memory, for pm_muon_step_noalloc).
 enum class TablePath { kStaged, kKernelArgs };
 
+// Tiles of one matrix in a stage (0 GRAM, 1 symmetric products, 2 UPDATE /
+// FINAL) at tile edge t; pad: of the padded extents.
+int32_t stage_tiles(const Plan& p, int st, int t, bool pad) {
+  if (t == kTile) return st < 2 ? sym_tiles(p) : full_tiles(p);
+  const int32_t m = pad ? p.Mp : p.M, n = pad ? p.Np : p.N;
+  return st < 2 ? mt_sym_tiles(m, t) : mt_full_tiles(m, n, t);
+}
+
+// The engine of one stage of a group.
+struct StageEngine {
+  int edge = kTile;         // kTile: the 256-tile engine, 128 or 64: the small-tile engine
+  bool persistent = false;  // small-tile engine: one block per CU, else one per item
+};
+
+// Chooses the tile of one stage of a group of engine matrices by its estimated
+// time in us. An item's time at a tile edge is an overhead plus its units of
+// 64 k; the coefficients are fits to per-launch times (rocprof) of lone and
+// grouped matrices from 256 x 256 to 5120 x 5120 and 4096 x 12288, measured at
+// all three edges, within some 15%. Bits do not depend on
+// the choice (the accumulation order of an element is the same at any edge).
+//   256: one round of n <= 256 items 17 + (0.85 + 0.85 n/256)·units, more
+//        rounds 11 + 1.4·units each (lone 1024 x 1024 product 30 us at 10
+//        items, 4096 x 4096 128 us at 256);
+//   128: 8 + 0.33·units alone, in rounds 4.5 + c·units, c growing with the
+//        operands' size as they leave the L2s;
+//    64: 5 + 0.12·units alone, (1.3 + 0.205·units)/256 each on a full chip
+//        (LDS reads bound it: half the FLOP per byte of 128).
+// The 256-tile engine keeps a stage unless a smaller tile is 5% ahead.
+StageEngine choose_engine(const Item* items, int count, int st) {
+  double n[3] = {0, 0, 0}, sum[3] = {0, 0, 0}, umax = 0, umin = 1e30;
+  constexpr int kEdge[3] = {kTile, 128, 64};
+  for (int i = 0; i < count; ++i) {
+    const Plan& p = items[i].plan;
+    const int ks = st == 0 ? p.ks_gram : st == 1 ? p.ks_symm : p.ks_full;
+    const double u = (double)(((st == 0 ? p.N : p.M) + 63) / 64) / ks;
+    const double c128 = 0.33 + 0.24 * p.Mp / 5120.0;
+    const double t[3] = {11 + 1.4 * u, 4.5 + c128 * u, 1.3 + 0.205 * u};
+    for (int e = 0; e < 3; ++e) {
+      const double k = (double)stage_tiles(p, st, kEdge[e], false) * ks;
+      n[e] += k;
+      sum[e] += k * t[e];
+    }
+    umax = std::max(umax, u);
+    umin = std::min(umin, u);
+  }
+  double est[3], r[3];
+  for (int e = 0; e < 3; ++e) r[e] = n[e] / 256;
+  est[0] = r[0] <= 1 ? 17 + (0.85 + 0.85 * r[0]) * umax
+                     : std::max(6 + sum[0] / 256 * std::ceil(r[0]) / r[0], 17 + 0.85 * umax);
+  est[1] = r[1] <= 1 ? 8 + 0.33 * umax
+                     : std::max(4 + sum[1] / 256 * (r[1] <= 2 ? 2 / r[1] : 1 + 0.35 / r[1]), 8 + 0.33 * umax);
+  est[2] = 3 + std::max(2 + 0.12 * umax, sum[2] / 256);
+  const int small = est[1] < est[2] ? 1 : 2;
+  if (est[small] > 0.95 * est[0]) return StageEngine{};
+  // 128-tiles run persistent when every item is as long as the next (a
+  // fixed share each); items of different lengths go one to a block
+  return StageEngine{kEdge[small], small == 1 && umin == umax};
+}
+
 int run_group(Item* items, int count, int group, const pm_hparams* hp, int mode, const float* lr_dev,
               double lr_host, char* ws, hipStream_t stream, TablePath path) {
   // plan_groups keeps small and engine matrices in separate groups: the engine's
@@ -644,6 +730,12 @@ int run_group(Item* items, int count, int group, const pm_hparams* hp, int mode,
       return fail(PM_EINVAL, "internal: a group mixes param dtypes");
 
   const int form = hp->ns_form;
+  StageEngine engine[3];
+  bool pad = false;  // some stage's 256-tile engine reads whole padded operands
+  for (int st = 0; st < 3 && !small; ++st) {
+    engine[st] = choose_engine(items, count, st);
+    pad = pad || engine[st].edge == kTile;
+  }
   // Table first, then per-matrix buffers.
   const size_t tb = table_bytes(count, gemm_launches(hp));
   char* cursor = ws + tb;
@@ -690,7 +782,8 @@ int run_group(Item* items, int count, int group, const pm_hparams* hp, int mode,
     cursor += p.kpart;
     descs[i] = d;
     pro[i + 1] = pro[i] + pro_tiles(p);
-    const int32_t tiles[3] = {sym_tiles(p), sym_tiles(p), full_tiles(p)};
+    const int32_t tiles[3] = {stage_tiles(p, 0, engine[0].edge, pad), stage_tiles(p, 1, engine[1].edge, pad),
+                              stage_tiles(p, 2, engine[2].edge, pad)};
     const int32_t ks[3] = {p.ks_gram, p.ks_symm, p.ks_full};
     for (int st = 0; st < 3; ++st) {
       const bool split = ks[st] > 1;
@@ -769,13 +862,15 @@ int run_group(Item* items, int count, int group, const pm_hparams* hp, int mode,
   L.ga.descs = ddesc;
   L.ga.n = count;
   L.ga.mode = mode;
+  L.ga.pad = pad;
   L.ga.lr_dev = lr_dev;
   L.ga.wd = (float)hp->weight_decay;
   L.ga.wdf_host = (float)(1.0 - lr_host * (double)hp->weight_decay);
   Launcher::Stage* sts[3] = {&L.gram_s, &L.sym_s, &L.full_s};
   for (int st = 0; st < 3; ++st)
     *sts[st] = Launcher::Stage{dev_ptr(pre[st][0]), dev_ptr(pre[st][1]), dev_ptr(pre[st][2]), pre[st][0][count],
-                               pre[st][1][count], pre[st][2][count]};
+                               pre[st][1][count], pre[st][2][count], engine[st].edge,
+                               engine[st].persistent};
   L.queues = dqueues;
   L.max_launches = gemm_launches(hp);
   L.final_f32 = mode == MODE_STEP && items[0].desc.p_dt == PM_DTYPE_F32;

@@ -96,6 +96,7 @@ struct GemmArgs {
   int32_t cur;            // which X ping-pong buffer holds the current X
   int32_t first;          // iteration 0: fold the Frobenius normalisation
   int32_t mode;
+  int32_t pad;             // small-tile engine: tiles cover the padded extents
   int32_t sl, sr, sd, sc;  // square-buffer operands: left, right, addend, output
   float a, b, c;           // UPDATE / FINAL: a; SYMM: alpha = c, beta = b
   const float* lr_dev;    // device lr, or null

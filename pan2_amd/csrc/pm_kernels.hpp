@@ -346,15 +346,17 @@ __device__ __forceinline__ void dma_b(const Engine& e, char* dst, int unit, int 
 // a+4, a+8 and a+12 of the group address, so source lane s points at row
 // k0 + 4h + s/4, columns c0 + 4(s%4) .. +3, and the two reads (h = 0, 1, four
 // rows = 512 bytes apart) return 4 consecutive k each.
-__device__ __forceinline__ bf16x8 tr_frag(const char* p) {
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ s16x4 tr_read(const char* p) {
   typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
-  const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 512));
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
+}
+__device__ __forceinline__ bf16x8 tr_pair(s16x4 v0, s16x4 v1) {
   typedef short s16x8 __attribute__((ext_vector_type(8)));
   const s16x8 w = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
   return __builtin_bit_cast(bf16x8, w);
 }
+__device__ __forceinline__ bf16x8 tr_frag(const char* p) { return tr_pair(tr_read(p), tr_read(p + 512)); }
 
 // Fragment j (16-row block of this wave's rows) of k-step s of the left
 // operand of unit buffer `buf`, and fragment j (16-column block) of the right.

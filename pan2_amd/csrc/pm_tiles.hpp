@@ -55,26 +55,26 @@ PM_HD void full_tile(int lt, int np, int nq, int& ti, int& tj) {
 // repeats: each panel comes from HBM about once instead of once per row group.
 constexpr int kGroupCols = 8;
 
-PM_HD void full_tile_cols(int lt, int np, int nq, int& ti, int& tj) {
+PM_HD void full_tile_cols(int lt, int np, int nq, int& ti, int& tj, int rows = kGroupRows) {
   const int per_cg = kGroupCols * np;  // tiles of a full column group
   const int cg = lt / per_cg;
   const int c0 = cg * kGroupCols;
   const int cw = imin(kGroupCols, nq - c0);
   const int r = lt - cg * per_cg;
-  const int rg = r / (kGroupRows * cw);
-  const int g0 = rg * kGroupRows;
-  const int gm = imin(kGroupRows, np - g0);
-  const int w = r - rg * kGroupRows * cw;
+  const int rg = r / (rows * cw);
+  const int g0 = rg * rows;
+  const int gm = imin(rows, np - g0);
+  const int w = r - rg * rows * cw;
   ti = g0 + w % gm;
   tj = c0 + w / gm;
 }
 
 // Upper triangle (ti <= tj) of an nt x nt tile grid, grouped the same way;
 // lt in [0, nt*(nt+1)/2).
-PM_HD void sym_tile(int lt, int nt, int& ti, int& tj) {
+PM_HD void sym_tile(int lt, int nt, int& ti, int& tj, int rows = kGroupRows) {
   int rem = lt, g0 = 0, gm = 0;
-  for (;; g0 += kGroupRows) {
-    gm = imin(kGroupRows, nt - g0);
+  for (;; g0 += rows) {
+    gm = imin(rows, nt - g0);
     const int cnt = gm * (gm + 1) / 2 + (nt - g0 - gm) * gm;
     if (rem < cnt) break;
     rem -= cnt;
@@ -121,6 +121,30 @@ PM_HD int k_split(int mp, int tiles, int kt) {
 PM_HD void split_item(int lt, int tiles, int& tile, int& chunk) {
   chunk = lt / tiles;
   tile = lt - chunk * tiles;
+}
+
+// Tiles of edge T that cover the first m rows (or columns) of a matrix, its
+// upper-triangle tiles, and the tiles of an m x n product: the small-tile
+// engine's (pm_mid.hpp), which leaves padding beyond the last tile alone.
+PM_HD int mt_edge_tiles(int m, int t) { return (m + t - 1) / t; }
+PM_HD int mt_sym_tiles(int m, int t) { return mt_edge_tiles(m, t) * (mt_edge_tiles(m, t) + 1) / 2; }
+PM_HD int mt_full_tiles(int m, int n, int t) { return mt_edge_tiles(m, t) * mt_edge_tiles(n, t); }
+
+// Work item of block b of a launch of n single-tile blocks (block b runs on
+// XCD b % 8): runs of up to RUN consecutive items per XCD, so the tiles
+// that share panels share an L2, the runs handed round robin so that long
+// items (first in the list) spread over the XCDs. A permutation of [0, n).
+template <int RUN>
+PM_HD int xcd_runs(int b, int n) {
+  constexpr int per = kXcds * RUN;
+  const int full = n / per * per;
+  if (b < full) {
+    const int w = b % per;
+    return b - w + (w % kXcds) * RUN + w / kXcds;
+  }
+  // the rest as eight runs whose lengths differ by one at most
+  const int r = n - full, w = b - full, x = w % kXcds;
+  return full + x * (r / kXcds) + imin(x, r % kXcds) + w / kXcds;
 }
 
 // Element offset of (r, c) in a workspace matrix with ld columns.
