@@ -511,7 +511,10 @@ struct Launcher {
   const float* coeffs = nullptr;  // device (a, b, c) per iteration
   int small_core(int cur, bool first, int it0, int steps, int it, bool r_in = false) {
     const SmallCoreArgs a{ga.descs, coeffs, it0, steps, cur, first, 0, r_in};
-    if (steps == 0)  // the standard form's M x M part fits a 4-slot ring: two blocks per CU
+    // the standard form's M x M part fits a 4-slot ring, so two blocks share a
+    // CU; with no second block to share it, the deeper ring's units in flight
+    // count (192 matrices of 128 x 4096: 52.5 -> 49.5 us a launch)
+    if (steps == 0 && count > gemm_grid(count))
       hipLaunchKernelGGL(pm_small_core_kernel<kSmRingStd>, dim3(count), dim3(kGemmThreads), 0, stream, a);
     else
       hipLaunchKernelGGL(pm_small_core_kernel<kSmRing>, dim3(count), dim3(kGemmThreads), 0, stream, a);
@@ -769,7 +772,9 @@ int run_group(Item* items, int count, int group, const pm_hparams* hp, int mode,
     const size_t x = align_up((size_t)p.Mp * p.Np * 2);
     const size_t a = align_up((size_t)p.Mp * p.Mp * 2);
     d.X[0] = (uint16_t*)cursor; cursor += x;
-    d.X[1] = (uint16_t*)cursor; cursor += x;
+    // a small matrix's apply updates X in place (each unit of X' depends on the
+    // same unit of X only, which its block has read into LDS)
+    d.X[1] = small ? d.X[0] : (uint16_t*)cursor; cursor += x;
     for (int b = 0; b < kSquareBufs; ++b) {
       d.S[b] = b < square_bufs(form, p.small) ? (uint16_t*)cursor : nullptr;
       if (b < square_bufs(form, p.small)) cursor += a;

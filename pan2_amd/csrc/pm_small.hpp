@@ -951,11 +951,13 @@ struct SmApply {
   static constexpr int kXCopies = kSmUnit / 1024 / kSmApplyWaves;
   static constexpr int kPCopies = kFinal ? kPBytes / 1024 / kSmApplyWaves : 0;
   static constexpr int kCopies = kXCopies + kPCopies;  // 1 KiB copies per unit and wave
-  static constexpr int kStores = 4;                    // vector stores per unit and wave
+  static constexpr int kStores = kFinal ? 4 : 2;       // vector stores per unit and wave
   // vmcnt while waiting for the r-th unit of the block: the copies of the
-  // kRing - 2 units issued after its own, and the stores of the units since
-  // (copies are issued right after each unit's barrier, its stores last)
-  static constexpr int kWaitMax = (kRing - 2) * kCopies + (kRing - 1) * kStores;
+  // kRing - 2 units issued after its own, and the stores of the units since.
+  // FINAL: a unit's copies right after its barrier, its stores last. UPDATE: a
+  // unit's X' is stored after the next unit's barrier, before its copies.
+  static constexpr int wait_at(int r) { return (kRing - 2) * kCopies + (kFinal ? r : r > 0 ? r - 1 : 0) * kStores; }
+  static constexpr int kWaitMax = wait_at(kRing - 1);
   static_assert(kWaitMax < 64, "vmcnt range");
   static_assert((kRing + (kFinal ? 0 : 2)) * kSmUnit + (kFinal ? kRing * kPBytes : 0) <= 160 * 1024, "LDS");
 };
@@ -965,7 +967,7 @@ template <class C, int R = 0>
 __device__ __forceinline__ void wait_unit(int r) {
   if constexpr (R < C::kRing - 1) {
     if (r == R) {
-      wait_vmcnt<(C::kRing - 2) * C::kCopies + R * C::kStores>();
+      wait_vmcnt<C::wait_at(R)>();
       return;
     }
     wait_unit<C, R + 1>(r);
@@ -1038,9 +1040,9 @@ __global__ __launch_bounds__(kSmApplyThreads, 1) void pm_small_apply_kernel(Gemm
     __shared__ __attribute__((aligned(1024))) char x7[kSmUnit];
     sl.x[4] = x4; sl.x[5] = x5; sl.x[6] = x6; sl.x[7] = x7;
   }
-  char* gt0 = nullptr;  // GRAM: X' of even / odd units, in the gram ring's layout
+  char* gt0 = nullptr;  // UPDATE: X' of even / odd units, in the gram ring's layout
   char* gt1 = nullptr;
-  if constexpr (GRAM) {
+  if constexpr (!kFinal) {
     __shared__ __attribute__((aligned(1024))) char gx0[kSmUnit];
     __shared__ __attribute__((aligned(1024))) char gx1[kSmUnit];
     gt0 = gx0;
@@ -1158,6 +1160,22 @@ __global__ __launch_bounds__(kSmApplyThreads, 1) void pm_small_apply_kernel(Gemm
   };
   const float wdf = step ? (args.lr_dev ? 1.0f - lr * args.wd : args.wdf_host) : 0.0f;
 
+  // UPDATE: a unit's X' goes through its LDS tile and out as whole rows (1 KiB
+  // of consecutive memory per store instruction) behind the next unit's
+  // barrier; xw: where the waiting unit's X' goes, or null. X is updated in
+  // place. Measured: 768 x 128 x 4096 with the gram 400 -> 365 us (32-byte
+  // pieces of rows before), 192 without 101 -> 88 (90 by the place alone: its
+  // 201 MB stay in the memory-side cache). Two blocks a CU on a 4-slot ring: 92.
+  uint16_t* xw = nullptr;
+  auto flush = [&](const char* gt) {
+    if (!xw) return;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int q = 2 * w + h, row = 8 * q + (lane >> 3);
+      const u32x4 v = lds_load16(gt + (q * 1024 + lane * 16));
+      glb_store16(xw + row * 64 + (((lane & 7) ^ ((row >> 1) & 7)) << 3), v);
+    }
+  };
   // GRAM: this wave's part of R (the core's layout), the unit whose X' waits
   // in its LDS tile, and the matrix whose last unit that is (-1: none)
   f32x4 gacc[4][2];
@@ -1198,8 +1216,9 @@ __global__ __launch_bounds__(kSmApplyThreads, 1) void pm_small_apply_kernel(Gemm
   // touching them.
   auto unit = [&](char* xs, const char* ps, char* nxs, char* nps, int u, char* gt, const char* gp) {
     wait_unit<C>(u - u0);
-    if constexpr (GRAM) wait_lgkmcnt<0>();  // this wave's X' tile writes of unit u-1 are done
+    if constexpr (!kFinal) wait_lgkmcnt<0>();  // this wave's X' tile writes of unit u-1 are done
     block_barrier();  // every wave's copies of u have landed; every wave is done with unit u-1
+    if constexpr (!kFinal) flush(gp);
     // unit u-1's X' is in its tile (written before the barrier); its gram, and
     // R of a finished matrix, before this unit's copies
     if constexpr (GRAM) gram_catch_up(gp);
@@ -1262,15 +1281,12 @@ __global__ __launch_bounds__(kSmApplyThreads, 1) void pm_small_apply_kernel(Gemm
       }
     }
     if constexpr (!kFinal) {
-      // X' row pr, columns n0 + q4 .. +3
-      uint16_t* xn = d.X[args.cur ^ 1] + sm_x_off(0, n0);
+      xw = d.X[args.cur ^ 1] + sm_x_off(0, n0);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
+        // row pr, columns q4 .. q4+3 of the unit, chunk q4/8 stored at (q4/8) ^ ((pr >> 1) & 7)
         const int pr = 64 * wr + 16 * i + 4 * g + (lane & 3), q4 = (16 * wc + r16) & ~3;
-        const u16x4 t = quad_transpose(o[i], lane);
-        *(u16x4*)(xn + pr * 64 + q4) = t;
-        // GRAM: row pr, columns q4 .. q4+3 of the unit, chunk q4/8 stored at (q4/8) ^ ((pr >> 1) & 7)
-        if constexpr (GRAM) *(u16x4*)(gt + pr * 128 + ((((q4 >> 3) ^ ((pr >> 1) & 7))) << 4) + (q4 & 7) * 2) = t;
+        *(u16x4*)(gt + (pr * 128 + ((((q4 >> 3) ^ ((pr >> 1) & 7))) << 4) + (q4 & 7) * 2)) = quad_transpose(o[i], lane);
       }
       if constexpr (GRAM) {
         gpend = true;
@@ -1367,10 +1383,12 @@ __global__ __launch_bounds__(kSmApplyThreads, 1) void pm_small_apply_kernel(Gemm
     }
   }
 #undef PM_SM_UNIT
-  if constexpr (GRAM) {
+  if constexpr (!kFinal) {
     wait_lgkmcnt<0>();
     block_barrier();  // every wave's X' of the block's last unit is in its tile
-    gram_catch_up(((u1 - 1 - u0) & 1) ? gt1 : gt0);
+    const char* last = ((u1 - 1 - u0) & 1) ? gt1 : gt0;
+    flush(last);
+    if constexpr (GRAM) gram_catch_up(last);
   }
   wait_vmcnt<0>();  // no copy is still writing this block's LDS when it ends
 }
