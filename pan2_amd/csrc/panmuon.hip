@@ -496,6 +496,20 @@ struct Launcher {
     a.stage = ST_SYMM; a.sl = sl; a.sr = sr; a.sd = sd; a.sc = sc; a.c = alpha; a.b = beta;
     return stage_launch<ST_SYMM, DT_BF16>(a, sym_s, PM_K_POLY, it, f_sym, "symmetric product launch");
   }
+  // S[sz] = alpha·S[sr]·S[sr] + beta·S[sr] and S[sq] = S[sz] + qa·I: the
+  // small-tile engine's epilogue writes both (two launches of 24-29 us less on
+  // a lone 1024 x 4096 and on a width-1024 block, 357 us at 15 matrices of
+  // width 5120); the 256-tile engine's stores are its epilogue's bound, and a
+  // second one there took as long as the copy
+  int symm_q(int sr, int sz, float alpha, float beta, int sq, float qa, int max_mp, int it) {
+    if (sym_s.edge == kTile) {
+      if (int rc = symm(sr, sr, sr, sz, alpha, beta, it)) return rc;
+      return qinit(sz, sq, qa, max_mp, it);
+    }
+    GemmArgs a = ga;
+    a.stage = ST_SYMM; a.sl = a.sr = a.sd = sr; a.sc = sz; a.c = alpha; a.b = beta; a.sq = sq; a.qa = qa;
+    return stage_launch<ST_SYMM, DT_BF16>(a, sym_s, PM_K_POLY, it, f_sym, "symmetric product launch");
+  }
   // X' = s·(a·X + S[sl]·X) into the other X slot, or (last) the param step
   int update(int sl, float coef_a, int cur, bool first, bool last, int it) {
     GemmArgs a = ga;
@@ -542,8 +556,8 @@ struct Launcher {
   }
   int qinit(int sz, int sq, float coef_a, int max_mp, int it) {
     for (int first = 0; first < count; first += 65535)  // gridDim.y limit
-      hipLaunchKernelGGL(pm_qinit_kernel, dim3(max_mp / kProTile, std::min(count - first, 65535)), dim3(kThreads), 0,
-                         stream, ga.descs, first, sz, sq, coef_a, (int32_t)((kWsLayout & kTiledS) != 0));
+      hipLaunchKernelGGL(pm_qinit_kernel, dim3(2 * (max_mp / kTile) * (max_mp / 64), std::min(count - first, 65535)),
+                         dim3(kThreads), 0, stream, ga.descs, first, sz, sq, coef_a);
     timing_mark(stream, PM_K_QINIT, group, it, count, 0.0, 0.0);
     return check("Q init launch");
   }
@@ -600,14 +614,14 @@ int run_gram(Launcher& L, const pm_hparams* hp, int max_mp) {
       if (!rc) rc = L.gram(cur, false, R, it);
       q = -1;
     }
-    if (!rc) rc = L.symm(R, R, R, Z, k.c, k.b, it);
     if (rc) break;
     if (q < 0) {
-      rc = L.qinit(Z, Q0, k.a, max_mp, it);
+      rc = L.symm_q(R, Z, k.c, k.b, Q0, k.a, max_mp, it);
       q = Q0;
     } else {
+      rc = L.symm(R, R, R, Z, k.c, k.b, it);
       const int qn = q == Q0 ? Q1 : Q0;
-      rc = L.symm(q, Z, q, qn, 1.0f, k.a, it);
+      if (!rc) rc = L.symm(q, Z, q, qn, 1.0f, k.a, it);
       q = qn;
     }
     if (!rc && it + 1 < steps && it + 1 != reset) {
@@ -868,6 +882,7 @@ int run_group(Item* items, int count, int group, const pm_hparams* hp, int mode,
   L.ga.n = count;
   L.ga.mode = mode;
   L.ga.pad = pad;
+  L.ga.sq = -1;
   L.ga.lr_dev = lr_dev;
   L.ga.wd = (float)hp->weight_decay;
   L.ga.wdf_host = (float)(1.0 - lr_host * (double)hp->weight_decay);

@@ -48,7 +48,7 @@ struct AdamArgs {
 __device__ __forceinline__ void adam_load8(const void* base, int32_t dt, int64_t off, bool vec, int valid,
                                            float (&v)[8]) {
   if (dt != DT_F16) {
-    load8(base, dt, off, vec, true, valid, v);
+    load8(base, dt, off, valid, v);
     return;
   }
   const _Float16* h = (const _Float16*)base + off;
@@ -66,7 +66,7 @@ __device__ __forceinline__ void adam_load8(const void* base, int32_t dt, int64_t
 __device__ __forceinline__ void adam_store8(void* base, int32_t dt, int64_t off, bool vec, int valid,
                                             const float (&v)[8]) {
   if (dt != DT_F16) {
-    store8(base, dt, off, vec, valid, v);
+    store8(base, dt, off, valid, v);
     return;
   }
   _Float16* h = (_Float16*)base + off;

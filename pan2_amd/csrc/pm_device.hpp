@@ -98,7 +98,9 @@ struct GemmArgs {
   int32_t mode;
   int32_t pad;             // small-tile engine: tiles cover the padded extents
   int32_t sl, sr, sd, sc;  // square-buffer operands: left, right, addend, output
+  int32_t sq;              // SYMM on the small-tile engine: S[sq] = S[sc] + qa·I as well (-1: no)
   float a, b, c;           // UPDATE / FINAL: a; SYMM: alpha = c, beta = b
+  float qa;
   const float* lr_dev;    // device lr, or null
   float wd;               // weight decay (device-lr path)
   float wdf_host;         // 1 - lr*wd (host-lr path)

@@ -6,6 +6,18 @@
 
 namespace pm {
 
+// A run of 8 bf16 elements with a added to element e (in fp32, rounded).
+__device__ __forceinline__ u32x4 add_diag(u32x4 v, int e, float a) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t lo = v[k] & 0xffffu, hi = v[k] >> 16;
+    const uint32_t qlo = f2bf(bf2f((uint16_t)lo) + a), qhi = f2bf(bf2f((uint16_t)hi) + a);
+    v[k] = (e == 2 * k ? qlo : lo) | ((e == 2 * k + 1 ? qhi : hi) << 16);
+  }
+  return v;
+}
+
 // ============================================================ prologue
 //
 // 64x64 tiles of the parameter, kProRun consecutive ones per block (tiles
@@ -19,23 +31,31 @@ namespace pm {
 // and partials[tile] = Σ bf16(u)², the tile's share of ‖X‖² (norm over the
 // bf16 tensor, torch/optim/_muon.py:59).
 // Each thread moves two runs of 8 consecutive elements of a row: 16-byte
-// loads and stores where the row is in range and the caller's strides and
-// bases allow, element by element otherwise. A transposed X goes through an
+// loads and stores (load8 / store8) of whole runs, element by element at a
+// row's end. A transposed X goes through an
 // LDS tile.
 constexpr int kProPitch = kProTile + 8;  // LDS row pitch (elements), keeps 16-byte rows aligned
 constexpr int kProRun = 4;  // tiles per prologue block, along a tile row (1 and 2 measured slower)
 static_assert(kTile % (kProTile * kProRun) == 0, "runs tile the padded long side");
 
-__device__ __forceinline__ void load8(const void* base, int32_t dt, int64_t off, bool vec, bool in_row, int valid,
-                                      float (&v)[8]) {
-  if (in_row && vec && valid >= 8) {
+// 16-byte vectors at any element's address: the hardware's unaligned access
+// mode, which the compiler targets on this platform, moves them in one
+// instruction (a row stride that is no multiple of 8 elements used to send
+// every run through element loads: three 777 x 1900 matrices' prologue 44 us,
+// now 23, and their FINAL 34, now 26).
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+
+// valid: how many of the 8 elements at base + off exist (<= 0: none)
+__device__ __forceinline__ void load8(const void* base, int32_t dt, int64_t off, int valid, float (&v)[8]) {
+  if (valid >= 8) {
     if (dt == DT_F32) {
-      const f32x4 a = *(const f32x4*)((const float*)base + off);
-      const f32x4 b = *(const f32x4*)((const float*)base + off + 4);
+      const f32x4 a = *(const f32x4_any*)((const float*)base + off);
+      const f32x4 b = *(const f32x4_any*)((const float*)base + off + 4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[4 + e] = b[e]; }
     } else {
-      const u32x4 a = *(const u32x4*)((const uint16_t*)base + off);
+      const u32x4 a = *(const u32x4_any*)((const uint16_t*)base + off);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         v[2 * e] = bf2f((uint16_t)(a[e] & 0xffff));
@@ -45,19 +65,19 @@ __device__ __forceinline__ void load8(const void* base, int32_t dt, int64_t off,
     return;
   }
 #pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = (in_row && e < valid) ? load_elem(base, dt, off + e) : 0.0f;
+  for (int e = 0; e < 8; ++e) v[e] = e < valid ? load_elem(base, dt, off + e) : 0.0f;
 }
 
-__device__ __forceinline__ void store8(void* base, int32_t dt, int64_t off, bool vec, int valid, const float (&v)[8]) {
-  if (vec && valid >= 8) {
+__device__ __forceinline__ void store8(void* base, int32_t dt, int64_t off, int valid, const float (&v)[8]) {
+  if (valid >= 8) {
     if (dt == DT_F32) {
-      *(f32x4*)((float*)base + off) = (f32x4){v[0], v[1], v[2], v[3]};
-      *(f32x4*)((float*)base + off + 4) = (f32x4){v[4], v[5], v[6], v[7]};
+      *(f32x4_any*)((float*)base + off) = (f32x4){v[0], v[1], v[2], v[3]};
+      *(f32x4_any*)((float*)base + off + 4) = (f32x4){v[4], v[5], v[6], v[7]};
     } else {
       u32x4 a;
 #pragma unroll
       for (int e = 0; e < 4; ++e) a[e] = (uint32_t)f2bf(v[2 * e]) | ((uint32_t)f2bf(v[2 * e + 1]) << 16);
-      *(u32x4*)((uint16_t*)base + off) = a;
+      *(u32x4_any*)((uint16_t*)base + off) = a;
     }
     return;
   }
@@ -92,8 +112,6 @@ __global__ __launch_bounds__(kThreads) void pm_prologue_kernel(ProArgs args) {
   const int ti = lt / nrun, tj0 = (lt - ti * nrun) * kProRun;  // first tile in X coordinates
   const float mu = args.mu, omu = 1.0f - args.mu;
   const bool step = args.mode == MODE_STEP;
-  const bool gvec = vec_ok(d.grad, d.g_dt, d.g_ld);
-  const bool mvec = step && vec_ok(d.mom, d.m_dt, d.m_ld);
   // X = u is written in the param's orientation (dst_a); X = uᵀ (a tall
   // param) goes through the LDS tile (dst_b). Only X is kept: the GEMM
   // engine reads it transposed where it needs Xᵀ.
@@ -117,21 +135,21 @@ __global__ __launch_bounds__(kThreads) void pm_prologue_kernel(ProArgs args) {
       const int r = (threadIdx.x >> 3) + 32 * h;
       const int pr = pr0 + r, pc = pc0 + cg;
       const bool in_row = pr < d.rows;
-      const int valid = d.cols - pc;  // elements of the run inside the parameter
+      const int valid = in_row ? d.cols - pc : 0;  // elements of the run inside the parameter
       float u[8];
       float g[8];
-      load8(d.grad, d.g_dt, (int64_t)pr * d.g_ld + pc, gvec, in_row, valid, g);
+      load8(d.grad, d.g_dt, (int64_t)pr * d.g_ld + pc, valid, g);
       if (step) {
         float m[8];
         const int64_t mo = (int64_t)pr * d.m_ld + pc;
-        load8(d.mom, d.m_dt, mo, mvec, in_row, valid, m);
+        load8(d.mom, d.m_dt, mo, valid, m);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float nm = mu * m[e] + omu * g[e];
           m[e] = nm;
           u[e] = args.nesterov ? omu * g[e] + mu * nm : nm;
         }
-        if (in_row) store8(d.mom, d.m_dt, mo, mvec, valid, m);
+        store8(d.mom, d.m_dt, mo, valid, m);
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) u[e] = g[e];
@@ -139,8 +157,8 @@ __global__ __launch_bounds__(kThreads) void pm_prologue_kernel(ProArgs args) {
       u32x4 packed;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const uint16_t lo = (in_row && 2 * e < valid) ? f2bf(u[2 * e]) : (uint16_t)0;
-        const uint16_t hi = (in_row && 2 * e + 1 < valid) ? f2bf(u[2 * e + 1]) : (uint16_t)0;
+        const uint16_t lo = 2 * e < valid ? f2bf(u[2 * e]) : (uint16_t)0;
+        const uint16_t hi = 2 * e + 1 < valid ? f2bf(u[2 * e + 1]) : (uint16_t)0;
         const float flo = bf2f(lo), fhi = bf2f(hi);
         ss += flo * flo;
         ss += fhi * fhi;
@@ -1617,28 +1635,31 @@ __global__ __launch_bounds__(64) void pm_ns_reduce_kernel(GemmArgs args) {
 // ============================================================ gram-form Q init
 // Q = Z + a·I for every matrix of the group: the first polynomial of a
 // gram-form segment, pan/optim/patch_muon.py:321-324 (Q = Z.clone(), then a
-// is added to the diagonal in bf16). Block (x, y) copies the 64-row band x of
-// matrix first + y; the padding rows and columns (beyond M) stay zero.
+// is added to the diagonal in bf16), for the stages that run on the 256-tile
+// engine (the small-tile engine's epilogue writes Q with Z). Block (x, y)
+// copies half a unit (128 rows x 64 columns, 16 consecutive KiB in the panel
+// layout) of matrix first + y; the padding (beyond M) stays zero. Bound by
+// HBM: 4 B per element read and written (blocks of 64 whole rows left a lone
+// 1024-wide matrix 16 blocks: 24 us).
 __global__ __launch_bounds__(kThreads) void pm_qinit_kernel(const MatDesc* descs, int32_t first, int32_t sz,
-                                                            int32_t sq, float a, int32_t tiled) {
+                                                            int32_t sq, float a) {
 #pragma clang fp contract(off)
   const MatDesc& d = descs[first + blockIdx.y];
-  const int r0 = blockIdx.x * kProTile;
-  if (r0 >= d.Mp) return;
-  const uint16_t* Z = d.S[sz];
-  uint16_t* Q = d.S[sq];
-  const int runs = d.Mp / 8;  // 16-byte runs per row
-  for (int i = threadIdx.x; i < kProTile * runs; i += kThreads) {
-    const int r = r0 + i / runs, c0 = (i % runs) * 8;
-    u32x4 v = *(const u32x4*)(Z + ws_off(r, c0, d.Mp, tiled));
-    const int e = r - c0;  // the diagonal element's place in this run, if any
-    if (r < d.M && e >= 0 && e < 8) {
-      const uint32_t w = v[e >> 1];
-      const uint16_t z = (e & 1) ? (uint16_t)(w >> 16) : (uint16_t)(w & 0xffffu);
-      const uint32_t q = f2bf(bf2f(z) + a);
-      v[e >> 1] = (e & 1) ? ((w & 0xffffu) | (q << 16)) : ((w & 0xffff0000u) | q);
-    }
-    *(u32x4*)(Q + ws_off(r, c0, d.Mp, tiled)) = v;
+  const int units = d.Mp / 64, x = blockIdx.x >> 1;  // unit x of the matrix: panel x / units, columns 64·(x % units)
+  if (x >= d.Mp / kTile * units) return;
+  const int r0 = x / units * kTile + 128 * (blockIdx.x & 1), c0 = x % units * 64;
+  const int64_t at = ((int64_t)x << 14) + ((blockIdx.x & 1) << 13);
+  const u32x4* Z = (const u32x4*)(d.S[sz] + at);
+  u32x4* Q = (u32x4*)(d.S[sq] + at);
+  u32x4 v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = Z[threadIdx.x + k * kThreads];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = threadIdx.x + k * kThreads, r = r0 + i / 8;
+    const int e = r - (c0 + i % 8 * 8);  // the diagonal element's place in this run, if any
+    if (r < d.M && e >= 0 && e < 8) v[k] = add_diag(v[k], e, a);
+    Q[i] = v[k];
   }
 }
 

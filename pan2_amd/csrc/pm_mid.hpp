@@ -333,11 +333,18 @@ __device__ __forceinline__ void mt_epilogue(const GemmArgs& args, const D& d, in
       uint16_t* C = d.S[args.sc];
       const float alpha = args.c;
       const int ld = d.Mp;
-      auto out = [&](const float (&x)[8], const u32x4& a, int64_t off) {
+      // the gram form's first Z of a segment also goes out as Q = Z + qa·I
+      const int sq = STAGE == ST_SYMM ? args.sq : -1;
+      uint16_t* Q = sq >= 0 ? d.S[sq] : nullptr;
+      // element (p, q) .. (p, q + 7)
+      auto out = [&](const float (&x)[8], const u32x4& a, int p, int q) {
         uint16_t o[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = f2bf(STAGE == ST_GRAM ? x[e] * s : alpha * x[e] + ca * at_el(a, e));
-        glb_store16(C + off, pack(o));
+        const int64_t off = ws_off(p, q, ld, true);
+        const u32x4 v = pack(o);
+        glb_store16(C + off, v);
+        if (sq >= 0) glb_store16(Q + off, diag && p < d.M && p >= q && p < q + 8 ? add_diag(v, p - q, args.qa) : v);
       };
 #pragma unroll
       for (int n = 0; n < kPasses; ++n) {
@@ -355,7 +362,7 @@ __device__ __forceinline__ void mt_epilogue(const GemmArgs& args, const D& d, in
             for (int e = 0; e < 8; ++e) x[e] = c + e < 64 * h + r ? y[e] : x[e];
           }
         }
-        out(x, an[h][n], ws_off(p0 + r, q0 + c, ld, true));
+        out(x, an[h][n], p0 + r, q0 + c);
       }
 #pragma unroll
       for (int n = 0; n < kPasses; ++n) {
@@ -363,7 +370,7 @@ __device__ __forceinline__ void mt_epilogue(const GemmArgs& args, const D& d, in
         if (diag && q < 64 * h + 64) continue;
         float x[8];
         col_run(p, q, x);
-        out(x, at[h][n], ws_off(q0 + q, p0 + p, ld, true));
+        out(x, at[h][n], q0 + q, p0 + p);
       }
     } else {
       // O of a row run: bf16((a·X + acc)·s)
@@ -398,7 +405,6 @@ __device__ __forceinline__ void mt_epilogue(const GemmArgs& args, const D& d, in
           block_barrier();
         }
         const int32_t dt = d.p_dt;
-        const bool vec = vec_ok(d.param, dt, d.p_ld);
         float p[kPasses][8];
         int row[kPasses], valid[kPasses];
         int64_t off[kPasses];
@@ -408,7 +414,7 @@ __device__ __forceinline__ void mt_epilogue(const GemmArgs& args, const D& d, in
           const int col = tall ? p0 + cc(n) : q0 + rc(n);
           valid[n] = row[n] < d.rows ? d.cols - col : 0;
           off[n] = (int64_t)row[n] * d.p_ld + col;
-          if (step) load8(d.param, dt, off[n], vec, valid[n] > 0, valid[n], p[n]);
+          if (step) load8(d.param, dt, off[n], valid[n], p[n]);
         }
 #pragma unroll
         for (int n = 0; n < kPasses; ++n) {
@@ -423,7 +429,7 @@ __device__ __forceinline__ void mt_epilogue(const GemmArgs& args, const D& d, in
           }
 #pragma unroll
           for (int e = 0; e < 8; ++e) f[e] = step ? p[n][e] * wdf + f[e] * neg : f[e];
-          if (valid[n] > 0) store8(d.param, dt, off[n], vec, valid[n], f);
+          store8(d.param, dt, off[n], valid[n], f);
         }
       }
     }
