@@ -323,11 +323,29 @@ def muon_step(params, grads, bufs, adj_ratios, *, lr, weight_decay, momentum, ne
     the library's static scratch (NOALLOC_SCRATCH_BYTES) with no workspace
     tensor; workspace_limit does not apply.
     """
-    lib = load()
     if len(params) == 0:
         return
-    dev = params[0].device
-    arr = _step_matrices(params, grads, bufs, adj_ratios, chunks)
+    muon_launch(_step_matrices(params, grads, bufs, adj_ratios, chunks), params[0].device, lr=lr,
+                weight_decay=weight_decay, momentum=momentum, nesterov=nesterov, ns_coefficients=ns_coefficients,
+                ns_steps=ns_steps, eps=eps, workspace_limit=workspace_limit, ns_form=ns_form, noalloc=noalloc)
+
+
+def muon_descs(params, grads, bufs, ratios, chunks: int):
+    """The pm_matrix array of one call (every param as ``chunks`` equal row
+    blocks, ratios[i] theirs), filled in one C++ pass, or None when some tensor
+    is not a plain contiguous float32 / bfloat16 matrix of its param's shape on
+    params[0]'s HIP device, is empty, or does not split into the row blocks."""
+    h = host_ext()
+    arr = np.empty(len(params) * chunks, dtype=_PM_MATRIX_NP)
+    rc = h.fill_muon(arr.ctypes.data, params, grads, bufs, ratios, chunks)
+    return arr if rc == h.FILLED else None
+
+
+def muon_launch(arr, dev, *, lr, weight_decay, momentum, nesterov, ns_coefficients, ns_steps, eps,
+                workspace_limit: int = 0, ns_form: str = "standard", noalloc: bool = False) -> None:
+    """pm_muon_step (or pm_muon_step_noalloc) over a filled pm_matrix array of
+    tensors on device dev, on its current stream."""
+    lib = load()
     n = len(arr)
     mats = arr.ctypes.data_as(ctypes.POINTER(PmMatrix))
     hp, keep = make_hparams(momentum=momentum, nesterov=nesterov, ns_coefficients=ns_coefficients,
@@ -364,7 +382,6 @@ def muon_step(params, grads, bufs, adj_ratios, *, lr, weight_decay, momentum, ne
 def newton_schulz_into(pairs, *, ns_coefficients=(3.4445, -4.7750, 2.0315), ns_steps=5, eps=1e-7,
                        workspace_limit: int = 0, ns_form: str = "standard") -> None:
     """pm_newton_schulz over [(input, output)] pairs; outputs are bf16, same shape."""
-    lib = load()
     n = len(pairs)
     if n == 0:
         return
@@ -380,6 +397,47 @@ def newton_schulz_into(pairs, *, ns_coefficients=(3.4445, -4.7750, 2.0315), ns_s
         m.rows, m.cols = x.shape
         m.in_ld, m.out_ld = _ld(x), _ld(o)
         m.in_dtype = dtype_code(x)
+    _ns_launch(mats, n, dev, ns_coefficients=ns_coefficients, ns_steps=ns_steps, eps=eps,
+               workspace_limit=workspace_limit, ns_form=ns_form)
+
+
+# numpy twin of PmNsMatrix: the matrices of a batch are filled as arrays
+_PM_NS_NP = np.dtype({
+    "names": [f for f, _ in PmNsMatrix._fields_],
+    "formats": ["u8", "u8", "i8", "i8", "i8", "i8", "i4", "i4"],
+    "offsets": [getattr(PmNsMatrix, f).offset for f, _ in PmNsMatrix._fields_],
+    "itemsize": ctypes.sizeof(PmNsMatrix),
+})
+
+
+def newton_schulz_batch(x: torch.Tensor, out: torch.Tensor, *, ns_coefficients=(3.4445, -4.7750, 2.0315),
+                        ns_steps=5, eps=1e-7, workspace_limit: int = 0, ns_form: str = "standard") -> None:
+    """pm_newton_schulz over the matrices of a contiguous [B, M, N] batch; out is
+    a contiguous bf16 batch of its shape (x itself, if that is bf16). The same
+    call as newton_schulz_into on its B pairs of slices, without the slices."""
+    if x.dim() != 3 or not x.is_contiguous() or not out.is_contiguous():
+        raise ValueError("newton_schulz_batch takes contiguous [B, M, N] tensors")
+    if not x.is_cuda or not out.is_cuda:
+        raise RuntimeError("newton_schulz_batch runs on HIP device tensors; libpanmuon has no CPU path")
+    if out.dtype != torch.bfloat16 or out.shape != x.shape:
+        raise ValueError("output must be bf16 and shaped like the input")
+    n, rows, cols = x.shape
+    if n == 0:
+        return
+    arr = np.zeros(n, dtype=_PM_NS_NP)
+    idx = np.arange(n, dtype=np.uint64)
+    for field, t in (("in_", x), ("out", out)):
+        arr[field] = np.uint64(t.data_ptr()) + idx * np.uint64(rows * cols * t.element_size())
+    arr["rows"], arr["cols"] = rows, cols
+    arr["in_ld"] = arr["out_ld"] = cols
+    arr["in_dtype"] = dtype_code(x)
+    _ns_launch(arr.ctypes.data_as(ctypes.POINTER(PmNsMatrix)), n, x.device, ns_coefficients=ns_coefficients,
+               ns_steps=ns_steps, eps=eps, workspace_limit=workspace_limit, ns_form=ns_form)
+    del arr
+
+
+def _ns_launch(mats, n: int, dev, *, ns_coefficients, ns_steps, eps, workspace_limit, ns_form) -> None:
+    lib = load()
     hp, keep = make_hparams(ns_coefficients=ns_coefficients, ns_steps=ns_steps, eps=eps,
                             workspace_limit=workspace_limit, ns_form=ns_form)
     with torch.cuda.device(dev):
@@ -499,7 +557,8 @@ _host = None
 
 def host_ext():
     """The _pm_host extension (pan2_amd/csrc/pm_host.cpp, built beside libpanmuon
-    by pan2_amd.build): fills pm_adam_tensor arrays from torch's tensor lists."""
+    by pan2_amd.build): fills pm_adam_tensor and pm_matrix arrays from torch's
+    tensor lists."""
     global _host
     if _host is None:
         try:
@@ -509,6 +568,9 @@ def host_ext():
         if _pm_host.DESC_BYTES != ctypes.sizeof(PmAdamTensor):
             raise RuntimeError(f"_pm_host's pm_adam_tensor is {_pm_host.DESC_BYTES} bytes, "
                                f"ctypes' {ctypes.sizeof(PmAdamTensor)}: rebuild")
+        if _pm_host.MATRIX_BYTES != ctypes.sizeof(PmMatrix):
+            raise RuntimeError(f"_pm_host's pm_matrix is {_pm_host.MATRIX_BYTES} bytes, "
+                               f"ctypes' {ctypes.sizeof(PmMatrix)}: rebuild")
         _host = _pm_host
     return _host
 

@@ -1,13 +1,16 @@
-// Host-side descriptor builder of the AdamW path (_pm_host, a CPython
-// extension compiled against torch's headers; no GPU call, no device code).
+// Host-side descriptor builders of the AdamW and Muon paths (_pm_host, a
+// CPython extension compiled against torch's headers; no GPU call, no device
+// code).
 //
-// torch's fused Adam is handed a param group's tensors as Python lists
-// (torch/optim/adam.py:803-898). Reading
-// each tensor's pointer, size and dtype from Python costs a method call per
-// attribute and tensor, most of the host time of a step over a few hundred
-// tensors; fill_adam reads them in one C++ pass and writes the pm_adam_tensor
-// array that pm_adam_step (include/panmuon.h) takes, checking on the way what
-// that entry point needs of the lists.
+// torch's fused Adam and its Muon step are handed a param group's tensors as
+// Python lists (torch/optim/adam.py:803-898, torch/optim/_muon.py:285-318).
+// Reading each tensor's pointer, size and dtype from Python costs a method
+// call per attribute and tensor, most of the host time of a step over many
+// tensors; fill_adam and fill_muon read them in one C++ pass and write the
+// descriptor array that pm_adam_step / pm_muon_step (include/panmuon.h) takes,
+// checking on the way what that entry point needs of the lists. (A step over
+// 30 weights of width 256: 415 us of host time with the Muon array filled from
+// Python, 153 with fill_muon, beside 168 us on the GPU.)
 #include <torch/extension.h>
 
 #include <cstdint>
@@ -92,14 +95,71 @@ int fill_adam(int64_t out, const std::vector<at::Tensor>& params, const std::vec
   return kFilled;
 }
 
+// A tensor the Muon step may take by pointer: a plain (not a subclass with its
+// own dispatch, as DTensor), contiguous fp32 or bf16 matrix on `dev`.
+bool muon_matrix(const at::Tensor& t, const c10::Device& dev) {
+  return !t.key_set().has(c10::DispatchKey::Python) && t.device() == dev && t.dim() == 2 && t.is_contiguous() &&
+         (t.scalar_type() == c10::ScalarType::Float || t.scalar_type() == c10::ScalarType::BFloat16);
+}
+
+// Fills the pm_matrix array at address `out` (params.size() * chunks entries)
+// from the lists of one Muon call: param i, its grad and momentum as `chunks`
+// equal row blocks, each with ratios[i]. Returns kFilled when every param, grad
+// and momentum buffer is a muon_matrix of one shape on params[0]'s HIP device,
+// not empty, its rows a multiple of chunks; kGeneral otherwise, lists of other
+// lengths included (the caller's checking loop says what is wrong or takes the
+// call another way; the array is complete only on kFilled). hip_only = false
+// also fills from CPU tensors, for the CPU tests of the array's layout.
+int fill_muon(int64_t out, const std::vector<at::Tensor>& params, const std::vector<at::Tensor>& grads,
+              const std::vector<at::Tensor>& bufs, const std::vector<double>& ratios, int64_t chunks, bool hip_only) {
+  const size_t n = params.size();
+  if (n == 0 || grads.size() != n || bufs.size() != n || ratios.size() != n || chunks < 1) return kGeneral;
+  TORCH_CHECK(out != 0, "fill_muon: null descriptor array");
+  auto* d = reinterpret_cast<pm_matrix*>(out);
+  const c10::Device dev = params[0].device();
+  if (hip_only && !dev.is_cuda()) return kGeneral;
+  for (size_t i = 0; i < n; ++i) {
+    const at::Tensor* t[3] = {&params[i], &grads[i], &bufs[i]};
+    for (const at::Tensor* x : t)
+      if (!muon_matrix(*x, dev) || x->sizes() != t[0]->sizes()) return kGeneral;
+    const int64_t rows = t[0]->size(0), cols = t[0]->size(1);
+    if (rows * cols == 0 || rows % chunks) return kGeneral;
+    char* at[3];
+    int64_t step[3];  // bytes from one row block to the next
+    for (int k = 0; k < 3; ++k) {
+      at[k] = static_cast<char*>(t[k]->data_ptr());
+      step[k] = rows / chunks * cols * t[k]->element_size();
+    }
+    for (int64_t c = 0; c < chunks; ++c) {
+      pm_matrix& e = *d++;
+      e.param = at[0] + c * step[0];
+      e.grad = at[1] + c * step[1];
+      e.momentum = at[2] + c * step[2];
+      e.rows = rows / chunks;
+      e.cols = cols;
+      e.param_ld = e.grad_ld = e.momentum_ld = cols;
+      e.param_dtype = dtype_code(t[0]->scalar_type());
+      e.grad_dtype = dtype_code(t[1]->scalar_type());
+      e.momentum_dtype = dtype_code(t[2]->scalar_type());
+      e.reserved = 0;
+      e.adj_ratio = ratios[i];
+    }
+  }
+  return kFilled;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.doc() = "pan2_amd host helpers: pm_adam_tensor descriptors from torch tensor lists";
+  m.doc() = "pan2_amd host helpers: pm_adam_tensor and pm_matrix descriptors from torch tensor lists";
+  m.def("fill_muon", &fill_muon, "Fill a pm_matrix array from Muon tensor lists", pybind11::arg("out"),
+        pybind11::arg("params"), pybind11::arg("grads"), pybind11::arg("bufs"), pybind11::arg("ratios"),
+        pybind11::arg("chunks"), pybind11::arg("hip_only") = true);
   m.def("fill_adam", &fill_adam, "Fill a pm_adam_tensor array from fused-Adam tensor lists", pybind11::arg("out"),
         pybind11::arg("params"), pybind11::arg("grads"), pybind11::arg("exp_avgs"), pybind11::arg("exp_avg_sqs"),
         pybind11::arg("max_exp_avg_sqs"), pybind11::arg("steps"), pybind11::arg("hip_only") = true);
   m.attr("FILLED") = static_cast<int>(kFilled);
   m.attr("GENERAL") = static_cast<int>(kGeneral);
   m.attr("DESC_BYTES") = static_cast<int>(sizeof(pm_adam_tensor));
+  m.attr("MATRIX_BYTES") = static_cast<int>(sizeof(pm_matrix));
 }

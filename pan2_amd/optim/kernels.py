@@ -76,6 +76,5 @@ def batched_gram_newtonschulz(X, ns_coefficients, ns_steps, eps, reset_iteration
     # the reference writes the result back into X when the batch reset (its
     # second segment ran), else returns a new tensor
     out = X if ns_steps > 2 else torch.empty_like(X)
-    _lib.newton_schulz_into([(X[i], out[i]) for i in range(X.shape[0])], ns_coefficients=ns_coefficients,
-                            ns_steps=ns_steps, eps=eps, ns_form="gram")
+    _lib.newton_schulz_batch(X, out, ns_coefficients=ns_coefficients, ns_steps=ns_steps, eps=eps, ns_form="gram")
     return out

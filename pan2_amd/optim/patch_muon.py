@@ -55,6 +55,26 @@ WORKSPACE_LIMIT = 0
 NS_FORM = "gram"
 
 
+def _group_descs(params, grads, bufs, base_adjust_lr_fn, chunks):
+    """The call's descriptor array when every tensor is a plain contiguous matrix
+    on one HIP device (_lib.muon_descs), else None. The lr ratio is that of a
+    row block's shape, looked up once per shape of the call."""
+    if not isinstance(chunks, int) or chunks < 1:
+        return None
+    by_shape: dict = {}
+    ratios = []
+    for p in params:
+        shape = p.shape
+        r = by_shape.get(shape)
+        if r is None:
+            if len(shape) != 2 or shape[0] % chunks or not p.is_cuda:
+                return None
+            r = _adjust_ratio(base_adjust_lr_fn, (shape[0] // chunks, shape[1]) if chunks > 1 else shape)
+            by_shape[shape] = r
+        ratios.append(r)
+    return _lib.muon_descs(params, grads, bufs, ratios, chunks)
+
+
 @torch.compiler.disable
 def _single_tensor_muon(
     params: list[Tensor],
@@ -90,6 +110,17 @@ def _single_tensor_muon(
         raise AssertionError("Chunking along dim 1 is not currently supported (previously supported without comm overlap)")
     if not params:
         return
+
+    # The common case, checked and turned into descriptors in one C++ pass; the
+    # loop below raises for what that pass does not take, or takes it apart
+    if nesterov:
+        arr = _group_descs(params, grads, muon_momentum_bufs, base_adjust_lr_fn,
+                           total_chunks if chunk_dim == 0 else 1)
+        if arr is not None:
+            _lib.muon_launch(arr, params[0].device, lr=lr, weight_decay=weight_decay, momentum=momentum,
+                             nesterov=nesterov, ns_coefficients=ns_coefficients, ns_steps=ns_steps, eps=eps,
+                             workspace_limit=WORKSPACE_LIMIT, ns_form=NS_FORM)
+            return
 
     p_list, g_list, b_list, ratios, counts = [], [], [], [], []
     for param, grad, buf in zip(params, grads, muon_momentum_bufs):
@@ -152,9 +183,8 @@ def newton_schulz(grad: Tensor, ns_coefficients, ns_steps: int, eps: float) -> T
         return out  # torch's NS returns an empty matrix unchanged in shape
     flat_in = x.reshape(-1, *x.shape[-2:])
     flat_out = out.view(-1, *x.shape[-2:])
-    _lib.newton_schulz_into([(flat_in[i], flat_out[i]) for i in range(flat_in.shape[0])],
-                            ns_coefficients=ns_coefficients, ns_steps=ns_steps, eps=eps,
-                            workspace_limit=WORKSPACE_LIMIT, ns_form=NS_FORM)
+    _lib.newton_schulz_batch(flat_in, flat_out, ns_coefficients=ns_coefficients, ns_steps=ns_steps, eps=eps,
+                             workspace_limit=WORKSPACE_LIMIT, ns_form=NS_FORM)
     return out
 
 
@@ -165,12 +195,14 @@ def patch_muon(ns_form: str | None = None) -> None:
     "gram" (the reference's production _gram_newtonschulz_local, the default)
     or "standard" (torch's quintic); None keeps the current choice
     (``NS_FORM``).
-    Loads libpanmuon first, so a missing or broken build fails here, loudly.
+    Loads libpanmuon and the _pm_host extension first, so a missing or broken
+    build fails here, loudly.
     """
     global NS_FORM
     if ns_form is not None:
         _lib.ns_form_code(ns_form)  # validates
         NS_FORM = ns_form
     _lib.load()
+    _lib.host_ext()
     torch.optim._muon._single_tensor_muon = _single_tensor_muon
     torch.optim._muon._zeropower_via_newtonschulz = newton_schulz
