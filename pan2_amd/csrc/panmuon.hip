@@ -1016,9 +1016,30 @@ int collect_ns(const pm_ns_matrix* mats, int n, int form, std::vector<Item>& ite
   return PM_OK;
 }
 
-int grid_for(int64_t n) {
-  const int64_t blocks = (n + kThreads - 1) / kThreads;
-  return (int)std::max<int64_t>(1, std::min<int64_t>(blocks, 256 * 64));
+// The elementwise kernels' launches, by the tensors' dtypes; kernels' grids
+// stay below 2^31 blocks for any tensor that fits the GPU.
+int64_t ew_blocks(int64_t n) { return (n + kEwBlock - 1) / kEwBlock; }
+
+template <bool B32, bool G32>
+void launch_momentum(bool u32, dim3 grid, hipStream_t stream, void* buf, const void* grad, void* update, int64_t n,
+                     float momentum, int32_t nesterov) {
+  if (u32)
+    hipLaunchKernelGGL((pm_momentum_kernel<B32, G32, true>), grid, dim3(kThreads), 0, stream, buf, grad, update, n,
+                       momentum, nesterov);
+  else
+    hipLaunchKernelGGL((pm_momentum_kernel<B32, G32, false>), grid, dim3(kThreads), 0, stream, buf, grad, update, n,
+                       momentum, nesterov);
+}
+
+template <bool P32>
+void launch_step(bool u32, dim3 grid, hipStream_t stream, void* param, const void* update, int64_t n,
+                 const float* lr_dev, float wd, float adj, float wdf, float neg) {
+  if (u32)
+    hipLaunchKernelGGL((pm_step_kernel<P32, true>), grid, dim3(kThreads), 0, stream, param, update, n, lr_dev, wd, adj,
+                       wdf, neg);
+  else
+    hipLaunchKernelGGL((pm_step_kernel<P32, false>), grid, dim3(kThreads), 0, stream, param, update, n, lr_dev, wd, adj,
+                       wdf, neg);
 }
 
 // ---- the allocation-free step's descriptor tables and scratch
@@ -1168,8 +1189,14 @@ int pm_momentum_nesterov(void* buf, int32_t buf_dtype, const void* grad, int32_t
   if (!buf || !grad || !update) return fail(PM_EINVAL, "NULL tensor pointer");
   if (!valid_dtype(buf_dtype) || !valid_dtype(grad_dtype) || !valid_dtype(update_dtype))
     return fail(PM_EDTYPE, "dtypes must be f32 or bf16");
-  hipLaunchKernelGGL(pm_momentum_kernel, dim3(grid_for(n)), dim3(kThreads), 0, (hipStream_t)stream, buf,
-                     buf_dtype, grad, grad_dtype, update, update_dtype, n, momentum, nesterov);
+  if (ew_blocks(n) > INT32_MAX) return fail(PM_EINVAL, "too many elements in one call");
+  const dim3 grid((uint32_t)ew_blocks(n));
+  const bool b32 = buf_dtype == PM_DTYPE_F32, g32 = grad_dtype == PM_DTYPE_F32, u32 = update_dtype == PM_DTYPE_F32;
+  const hipStream_t s = (hipStream_t)stream;
+  if (b32 && g32) launch_momentum<true, true>(u32, grid, s, buf, grad, update, n, momentum, nesterov);
+  else if (b32) launch_momentum<true, false>(u32, grid, s, buf, grad, update, n, momentum, nesterov);
+  else if (g32) launch_momentum<false, true>(u32, grid, s, buf, grad, update, n, momentum, nesterov);
+  else launch_momentum<false, false>(u32, grid, s, buf, grad, update, n, momentum, nesterov);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? PM_OK : hip_fail(e, "momentum launch");
 }
@@ -1183,8 +1210,13 @@ int pm_step_param(void* param, int32_t param_dtype, const void* update, int32_t 
   if (!valid_dtype(param_dtype) || !valid_dtype(update_dtype)) return fail(PM_EDTYPE, "dtypes must be f32 or bf16");
   const float wdf = (float)(1.0 - lr_host * (double)weight_decay);
   const float neg = (float)(-(lr_host * adj_ratio));
-  hipLaunchKernelGGL(pm_step_kernel, dim3(grid_for(n)), dim3(kThreads), 0, (hipStream_t)stream, param,
-                     param_dtype, update, update_dtype, n, lr_dev, weight_decay, (float)adj_ratio, wdf, neg);
+  if (ew_blocks(n) > INT32_MAX) return fail(PM_EINVAL, "too many elements in one call");
+  const dim3 grid((uint32_t)ew_blocks(n));
+  const bool u32 = update_dtype == PM_DTYPE_F32;
+  if (param_dtype == PM_DTYPE_F32)
+    launch_step<true>(u32, grid, (hipStream_t)stream, param, update, n, lr_dev, weight_decay, (float)adj_ratio, wdf, neg);
+  else
+    launch_step<false>(u32, grid, (hipStream_t)stream, param, update, n, lr_dev, weight_decay, (float)adj_ratio, wdf, neg);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? PM_OK : hip_fail(e, "step launch");
 }
