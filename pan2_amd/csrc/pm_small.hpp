@@ -84,11 +84,6 @@ __device__ __forceinline__ char* sm_at(const SmMat& m, int half, int rr, int c16
   // scratch memory and reload the base from there on every access
   return (half ? m.h1 : m.h0) + rr * kSmRow + ((c16 ^ (rr & 15)) << 4);
 }
-// element (64·half + rr, q)
-__device__ __forceinline__ uint16_t* sm_el(const SmMat& m, int half, int rr, int q) {
-  return (uint16_t*)(sm_at(m, half, rr, q >> 3) + (q & 7) * 2);
-}
-
 // 16-byte LDS accesses through a pointer the compiler may only know as
 // generic (an LDS matrix picked at run time): the cast keeps them ds_
 // instructions rather than flat ones, which would also count in vmcnt.
@@ -105,98 +100,189 @@ __device__ __forceinline__ f32x4 mfma_bf16(const bf16x8& a, const bf16x8& b, con
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// Stores elements e of v with p0 + e < q: the strict lower part of row q,
-// columns p0 .. p0+3 (v[e] is the element at column p0 + e).
-__device__ __forceinline__ void store_lower4(uint16_t* dst, u16x4 v, int p0, int q) {
-  if (p0 + 3 < q) {
-    *(u16x4*)dst = v;
-    return;
-  }
-  if (p0 >= q) return;
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    if (p0 + e < q) dst[e] = v[e];
+// A 128 x 128 LDS matrix of the core kernel by address, so that one body of
+// code serves every product (the operands are picked at run time): rows 0..63
+// at h0, rows 64..127 at h0 + d, laid out as SmMat's halves.
+struct SmRef {
+  uint32_t h0, d;
+};
+__device__ __forceinline__ uint32_t sm_lds_addr(const char* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
+}
+__device__ __forceinline__ SmRef sm_ref(const SmMat& m) { return SmRef{sm_lds_addr(m.h0), sm_lds_addr(m.h1) - sm_lds_addr(m.h0)}; }
+// byte address of element (r, q)
+__device__ __forceinline__ uint32_t sm_ref_at(const SmRef& m, int r, int q) {
+  return m.h0 + (r >> 6) * m.d + (r & 63) * kSmRow + (((q >> 3) ^ (r & 15)) << 4) + (q & 7) * 2;
+}
+template <class V>
+__device__ __forceinline__ __attribute__((address_space(3))) V* sm_ref_ptr(uint32_t at) {
+  return (__attribute__((address_space(3))) V*)(uintptr_t)at;
 }
 
-// Finishes a 128 x 128 product of 8 waves, wave w owning rows r0 .. r0+63
-// (r0 = 64·(w/4)) and columns c0 .. c0+31 (c0 = 32·(w%4)); acc[i][j] holds
-// rows r0 + 16i + 4(lane/16) + 0..3 of column c0 + 16j + lane%16.
-// C = alpha·acc + beta·D, rounded to bf16; elements on and above the diagonal
-// are stored at (p, q) and (q, p), so C is exactly symmetric. D must be
-// symmetric (it is read through its transpose). C may be an operand of the
-// product: every wave has read its operands before the first store.
-__device__ __forceinline__ void sm_finish(const f32x4 (&acc)[4][2], const SmMat& D, const SmMat& C, float alpha,
-                                          float beta, int r0, int c0, int lane) {
+// A product's waves: wave w owns the 64 x 32 block sm_block(w) of C (rows
+// 64·(b/4), columns 32·(b%4)). Elements below the diagonal are neither stored
+// nor mirrored, so blocks 4 and 5 are idle and the others hold 3, 7, 8, 8, -, -,
+// 3, 7 of their 8 tiles of 16 x 16: waves w and w + 4 share a SIMD, and this
+// order gives the four SIMDs 8, 8, 10 and 10 tiles (in block order 3 to 15).
+__device__ __forceinline__ int sm_block(int w) { return (0x60547132 >> (4 * w)) & 15; }
+__device__ __forceinline__ bool sm_idle(int r0, int c0) { return r0 > c0 + 31; }
+
+// Lane parts of the byte addresses a product uses, with the chunk swizzle
+// (sm_ref_at) split so that a tile's address is the part of its row block, a
+// lane offset and one XOR: rows rb + 4(lane/16) + lane%4, columns cb +
+// (lane%16 & ~3) .. +3 at base(rb) + up + ((2·cb) ^ upx); row cb + lane%16,
+// columns rb + 4(lane/16) .. +3 at base(cb) + lo + ((2·rb) ^ lox); the MFMA
+// fragment of rows rb + lane%16, k = 32s + 8(lane/16) .. +7 at base(rb) + fr[s]
+// (rb, cb multiples of 16). A product is bound by the VALU instructions of its
+// 36 tiles and the LDS reads of its operands; with addresses formed per access
+// it took 4550 cycles, 1900-2250 of them the masked stores. The core launches
+// of a lone matrix of 1 x 320 now take 21 us (26.4 before), of 768 x 128 x 4096
+// 62 us (75 before).
+struct SmLane {
+  int up, upx, lo, lox, fr[4];
+};
+__device__ __forceinline__ SmLane sm_lane(int lane) {
+  const int r16 = lane & 15, g = lane >> 4, rl = 4 * g + (lane & 3);
+  SmLane k;
+  k.up = rl * kSmRow + (r16 & 4) * 2;
+  k.upx = ((r16 >> 3) ^ rl) << 4;
+  k.lo = r16 * kSmRow + (g & 1) * 8;
+  k.lox = ((g >> 1) ^ r16) << 4;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) k.fr[s] = r16 * kSmRow + (((4 * s + g) ^ r16) << 4);
+  return k;
+}
+__device__ __forceinline__ uint32_t sm_row_base(const SmRef& m, int rb) {
+  return m.h0 + (rb >> 6) * m.d + (rb & 63) * kSmRow;
+}
+
+// The addend D[p0..p0+3][q] of a wave's tiles (above or on the diagonal only;
+// D is symmetric, so it is read through its transpose).
+__device__ __forceinline__ void sm_addend(u16x4 (&dv)[4][2], const SmRef& D, float beta, int r0, int c0,
+                                          const SmLane& k) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int rb = r0 + 16 * i, cb = c0 + 16 * j;
+      dv[i][j] = (u16x4){0, 0, 0, 0};
+      if (beta != 0.0f && cb >= rb) dv[i][j] = *sm_ref_ptr<const u16x4>(sm_row_base(D, cb) + k.lo + ((2 * rb) ^ k.lox));
+    }
+}
+
+// A wave's 64 x 32 block of C = alpha·acc + beta·D, rounded to bf16 (acc[i][j]:
+// rows r0 + 16i + 4(lane/16) + 0..3 of column c0 + 16j + lane%16, dv the addend
+// there), as the pieces sm_put stores: o the quads, t the same turned into
+// pieces of rows. C is exactly symmetric: a 16 x 16 tile above the diagonal
+// goes whole to both places, one below it nowhere, the diagonal's own once,
+// each row's part left of the diagonal taken from the lanes that hold its
+// mirror (masked stores of it took as long as four whole tiles).
+struct SmPieces {
+  u16x4 o[4][2], t[4][2];
+};
+__device__ __forceinline__ void sm_turn(SmPieces& w, const f32x4 (&acc)[4][2], const u16x4 (&dv)[4][2], float alpha,
+                                        float beta, int r0, int c0, int lane) {
 #pragma clang fp contract(off)
-  const int g = lane >> 4;
-  const int rh = r0 >> 6, ch = c0 >> 6, cr = c0 & 63;  // halves and row-in-half base of the wave
-  u16x4 o[4][2];
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int p0 = r0 + 16 * i + 4 * g;
-      u16x4 dv = (u16x4){0, 0, 0, 0};
-      if (beta != 0.0f) dv = *(const u16x4*)sm_el(D, ch, cr + 16 * j + (lane & 15), p0);  // D[p0..p0+3][q]
+      const int rb = r0 + 16 * i, cb = c0 + 16 * j;  // wave-uniform corner of the tile
+      w.o[i][j] = w.t[i][j] = (u16x4){0, 0, 0, 0};
+      if (cb < rb) continue;
+      u16x4 o;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[i][j][r] = f2bf(alpha * acc[i][j][r] + beta * bf2f(dv[r]));
+      for (int r = 0; r < 4; ++r) o[r] = f2bf(alpha * acc[i][j][r] + beta * bf2f(dv[i][j][r]));
+      u16x4 t = quad_transpose(o, lane);
+      if (cb == rb) {
+        // row p = 4(lane/16) + lane%4, columns q4 .. q4+3 (q4 = lane & 12): the
+        // mirror of the row's part left of p is rows q4 .. q4+3 of column p, the
+        // quad of lane 4·q4 + p
+        const int p = 4 * (lane >> 4) + (lane & 3), q4 = lane & 12, src = (4 * q4 + p) * 4;
+        const u32x2 v = __builtin_bit_cast(u32x2, o);
+        const u32x2 mv = {(uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)v.x),
+                          (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)v.y)};
+        const u16x4 mr = __builtin_bit_cast(u16x4, mv);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[e] = q4 + e >= p ? t[e] : mr[e];
+      }
+      w.o[i][j] = o;
+      w.t[i][j] = t;
     }
+}
+__device__ __forceinline__ void sm_put(const SmPieces& w, const SmRef& C, int r0, int c0, const SmLane& k) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int rb = r0 + 16 * i, cb = c0 + 16 * j;
+      if (cb < rb) continue;
+      // row p, columns q4 .. q4+3, and the mirror: row q, columns p0 .. p0+3
+      *sm_ref_ptr<u16x4>(sm_row_base(C, rb) + k.up + ((2 * cb) ^ k.upx)) = w.t[i][j];
+      if (cb > rb) *sm_ref_ptr<u16x4>(sm_row_base(C, cb) + k.lo + ((2 * rb) ^ k.lox)) = w.o[i][j];
+    }
+}
+
+// Finishes a 128 x 128 product of 8 waves (sm_block). C may be an operand of
+// the product: every wave has read its operands before the first store, and
+// does everything but the stores before that barrier.
+__device__ __forceinline__ void sm_finish(const f32x4 (&acc)[4][2], const u16x4 (&dv)[4][2], const SmRef& C,
+                                          float alpha, float beta, int r0, int c0, const SmLane& k, int lane) {
+  SmPieces w;
+  sm_turn(w, acc, dv, alpha, beta, r0, c0, lane);
   __syncthreads();  // every wave has read its operands and D
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int p0 = r0 + 16 * i + 4 * g, q = c0 + 16 * j + (lane & 15);
-      // row p0 + lane%4, columns q&~3 .. +3 (quad_transpose), on and above the diagonal
-      const u16x4 t = quad_transpose(o[i][j], lane);
-      store_upper4(sm_el(C, rh, 16 * i + 4 * g + (lane & 3), q & ~3), t, q & ~3, p0 + (lane & 3));
-      // the mirror: row q, columns p0 .. p0+3, strictly below the diagonal
-      store_lower4(sm_el(C, ch, cr + 16 * j + (lane & 15), p0), o[i][j], p0, q);
-    }
+  sm_put(w, C, r0, c0, k);
   __syncthreads();
 }
 
-// Waves 4 and 5 own rows 64..127 of columns 0..63: every element of their
-// tiles lies below the diagonal, which sm_finish neither stores nor mirrors, so
-// they skip the products (fragment reads and MFMAs) and only keep the block's
-// barriers.
-__device__ __forceinline__ bool sm_idle(int r0, int c0) { return r0 > c0 + 31; }
-
 // C = alpha·L·Rᵀ + beta·D on 128 x 128 LDS matrices (K = 128). Every matrix
 // here is symmetric, so L Rᵀ = L R.
-__device__ __forceinline__ void sm_product(const SmMat& L, const SmMat& R, const SmMat& D, const SmMat& C, float alpha,
-                                           float beta, int wave, int lane) {
-  const int r0 = (wave >> 2) * 64, c0 = (wave & 3) * 32;
-  const int r16 = lane & 15, g = lane >> 4;
+template <int BATCH>
+__device__ __forceinline__ void sm_product(const SmRef& L, const SmRef& R, const SmRef& D, const SmRef& C, float alpha,
+                                           float beta, int r0, int c0, const SmLane& k, int lane) {
   f32x4 acc[4][2];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  u16x4 dv[4][2];
+  sm_addend(dv, D, beta, r0, c0, k);
   if (!sm_idle(r0, c0)) {
+    // the fragments of BATCH k-steps are requested before their first MFMA
+    // (left to itself the compiler reads two or three, waits, and pays the LDS
+    // latency each time); two blocks a CU leave registers for two k-steps
+    const uint32_t lb = sm_row_base(L, r0), rb = sm_row_base(R, c0);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {  // k = 32s .. 32s+31: logical chunks 4s .. 4s+3
-      bf16x8 a[4], b[2];
+    for (int s0 = 0; s0 < 4; s0 += BATCH) {  // k = 32s .. 32s+31
+      bf16x8 a[BATCH][4], b[BATCH][2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = *(const bf16x8*)sm_at(L, r0 >> 6, 16 * i + r16, 4 * s + g);
+      for (int s = 0; s < BATCH; ++s) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = *(const bf16x8*)sm_at(R, c0 >> 6, (c0 & 63) + 16 * j + r16, 4 * s + g);
+        for (int i = 0; i < 4; ++i) a[s][i] = *sm_ref_ptr<const bf16x8>(lb + k.fr[s0 + s] + i * 16 * kSmRow);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int j = 0; j < 2; ++j) b[s][j] = *sm_ref_ptr<const bf16x8>(rb + k.fr[s0 + s] + j * 16 * kSmRow);
+      }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = mfma_bf16(a[i], b[j], acc[i][j]);
+      for (int s = 0; s < BATCH; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = mfma_bf16(a[s][i], b[s][j], acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
-  sm_finish(acc, D, C, alpha, beta, r0, c0, lane);
+  sm_finish(acc, dv, C, alpha, beta, r0, c0, k, lane);
 }
 
 // Q = Z + a·I on the first m rows (pan/optim/patch_muon.py:321-324: the
 // diagonal add in bf16); the padding rows and columns stay zero.
-__device__ __forceinline__ void sm_qinit(const SmMat& Z, const SmMat& Q, float a, int m) {
+__device__ __forceinline__ void sm_qinit(const SmRef& Z, const SmRef& Q, float a, int m) {
 #pragma clang fp contract(off)
   for (int i = threadIdx.x; i < kSm * kSm / 8; i += blockDim.x) {
     const int r = i >> 4, c = i & 15;  // logical chunk c of row r: columns 8c .. 8c+7
-    u32x4 v = *(const u32x4*)sm_at(Z, r >> 6, r & 63, c);
+    u32x4 v = *sm_ref_ptr<const u32x4>(sm_ref_at(Z, r, 8 * c));
     const int e = r - 8 * c;  // the diagonal element's position in the chunk
     if (r < m && e >= 0 && e < 8) {
       const uint32_t w = v[e >> 1];
@@ -204,7 +290,7 @@ __device__ __forceinline__ void sm_qinit(const SmMat& Z, const SmMat& Q, float a
       const uint32_t qv = f2bf(bf2f(z) + a);
       v[e >> 1] = (e & 1) ? ((w & 0xffffu) | (qv << 16)) : ((w & 0xffff0000u) | qv);
     }
-    *(u32x4*)sm_at(Q, r >> 6, r & 63, c) = v;
+    *sm_ref_ptr<u32x4>(sm_ref_at(Q, r, 8 * c)) = v;
   }
   __syncthreads();
 }
@@ -252,19 +338,23 @@ struct SmCopy {
 __device__ __forceinline__ void sm_gram_acc(const char* src, f32x4 (&acc)[4][2], int r0, int c0, int lane) {
   if (sm_idle(r0, c0)) return;
   const int r16 = lane & 15, g = lane >> 4;
+  // the unit's fragments are requested before its first MFMA (as in sm_product)
+  bf16x8 a[2][4], b[2][2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     const int fo = r16 * 128 + (((4 * s + g) ^ ((r16 >> 1) & 7)) << 4);
-    bf16x8 a[4], b[2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) a[i] = *(const bf16x8*)(src + (r0 + 16 * i) * 128 + fo);
+    for (int i = 0; i < 4; ++i) a[s][i] = *(const bf16x8*)(src + ((r0 + 16 * i) * 128 + fo));
 #pragma unroll
-    for (int j = 0; j < 2; ++j) b[j] = *(const bf16x8*)(src + (c0 + 16 * j) * 128 + fo);
+    for (int j = 0; j < 2; ++j) b[s][j] = *(const bf16x8*)(src + ((c0 + 16 * j) * 128 + fo));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = mfma_bf16(a[i], b[j], acc[i][j]);
-  }
+      for (int j = 0; j < 2; ++j) acc[i][j] = mfma_bf16(a[s][i], b[s][j], acc[i][j]);
 }
 
 // R = bf16(alpha·acc) written row-major (128 x 128) to global memory, through
@@ -277,27 +367,12 @@ __device__ __forceinline__ void sm_gram_acc(const char* src, f32x4 (&acc)[4][2],
 // __syncthreads fence would also wait for the copies in flight.
 __device__ __forceinline__ void sm_gram_store(uint16_t* Rg, const SmMat& T, const f32x4 (&acc)[4][2], int r0, int c0,
                                               int lane, float alpha = 1.0f) {
-#pragma clang fp contract(off)
-  const int g = lane >> 4;
-  const int rh = r0 >> 6, ch = c0 >> 6, cr = c0 & 63;
-  const float beta = 0.0f;
-  u16x4 o[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[i][j][r] = f2bf(alpha * acc[i][j][r] + beta * bf2f((uint16_t)0));
+  const SmLane k = sm_lane(lane);
+  const u16x4 none[4][2] = {};
+  SmPieces w;
+  sm_turn(w, acc, none, alpha, 0.0f, r0, c0, lane);
   block_barrier();
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int p0 = r0 + 16 * i + 4 * g, q = c0 + 16 * j + (lane & 15);
-      store_upper4(sm_el(T, rh, 16 * i + 4 * g + (lane & 3), q & ~3), quad_transpose(o[i][j], lane), q & ~3,
-                   p0 + (lane & 3));
-      store_lower4(sm_el(T, ch, cr + 16 * j + (lane & 15), p0), o[i][j], p0, q);
-    }
+  sm_put(w, sm_ref(T), r0, c0, k);
   wait_lgkmcnt<0>();
   block_barrier();
   for (int i = threadIdx.x; i < kSm * kSm / 8; i += blockDim.x) {
@@ -349,8 +424,9 @@ __global__ __launch_bounds__(kGemmThreads, kSmRing / RING) void pm_small_core_ke
   }
 
   const MatDesc& d = args.descs[blockIdx.x];
-  const int wave = wave_id(), lane = lane_id();
-  const int r0 = (wave >> 2) * 64, c0 = (wave & 3) * 32;
+  const int wave = wave_id(), lane = threadIdx.x & 63;
+  const int blk = sm_block(wave), r0 = (blk >> 2) * 64, c0 = (blk & 3) * 32;
+  const SmLane k = sm_lane(lane);
 
   if (args.r_in) {
     // ---- R from S[so], where the apply that produced X stored it
@@ -405,37 +481,47 @@ __global__ __launch_bounds__(kGemmThreads, kSmRing / RING) void pm_small_core_ke
     // R = s²·X Xᵀ (s² = 1/‖X‖² on the unscaled first X): sm_finish's first
     // barrier also ends every wave's reads of the ring, whose first two slots
     // R overwrites (every copy has landed: the last unit waited for all)
-    sm_finish(acc, R, R, args.first ? d.scales[0] : 1.0f, 0.0f, r0, c0, lane);
+    const u16x4 none[4][2] = {};
+    sm_finish(acc, none, sm_ref(R), args.first ? d.scales[0] : 1.0f, 0.0f, r0, c0, k, lane);
   }
 
-  // ---- the M x M part of the iteration
-  bool out_q = false;  // S = Z (standard form) or Q (gram form)
+  // ---- the M x M part of the iteration: a list of products run by one body
+  // (inlined once a product it is 70 KB of code)
+  const SmRef mR = sm_ref(R), mZ = sm_ref(Z);
+  SmRef mS = mZ;  // S = Z (standard form) or Q (gram form)
   if (RING == kSmRingStd || args.steps == 0) {
-    const float* k = args.coeffs + 3 * args.it0;
-    sm_product(R, R, R, Z, k[2], k[1], wave, lane);  // B = c R R + b R
+    const float* co = args.coeffs + 3 * args.it0;
+    sm_product<RING == kSmRing ? 4 : 2>(mR, mR, mR, mZ, co[2], co[1], r0, c0, k, lane);  // B = c R R + b R
   } else if constexpr (RING == kSmRing) {
+    const SmRef mQ = sm_ref(Q), mRZ = sm_ref(RZ);
+    auto pick = [](bool c, const SmRef& x, const SmRef& y) { return SmRef{c ? x.h0 : y.h0, c ? x.d : y.d}; };
+    const int m = d.M;
     for (int i = 0; i < args.steps; ++i) {
-      const float* k = args.coeffs + 3 * (args.it0 + i);
-      const float a = k[0], b = k[1], c = k[2];
-      sm_product(R, R, R, Z, c, b, wave, lane);  // Z = c R R + b R
-      if (i == 0)
-        sm_qinit(Z, Q, a, d.M);  // Q = a I + Z
-      else
-        sm_product(Q, Z, Q, Q, 1.0f, a, wave, lane);  // Q = Q Z + a Q
-      if (i + 1 < args.steps) {
-        sm_product(R, Z, R, RZ, 1.0f, a, wave, lane);   // RZ = R Z + a R
-        sm_product(Z, RZ, RZ, R, 1.0f, a, wave, lane);  // R = Z RZ + a RZ
+      const float* co = args.coeffs + 3 * (args.it0 + i);
+      const float a = co[0], b = co[1], c = co[2];
+      // op 0: Z = c R R + b R;  1: Q = a I + Z (first), then Q = Q Z + a Q;
+      // unless the segment ends, 2: RZ = R Z + a R;  3: R = Z RZ + a RZ
+#pragma unroll 1
+      for (int op = 0; op < (i + 1 < args.steps ? 4 : 2); ++op) {
+        if (op == 1 && i == 0) {
+          sm_qinit(mZ, mQ, a, m);
+          continue;
+        }
+        const SmRef L = pick(op == 1, mQ, pick(op == 3, mZ, mR));
+        const SmRef rt = pick(op == 0, mR, pick(op == 3, mRZ, mZ));
+        const SmRef D = pick(op == 1, mQ, pick(op == 3, mRZ, mR));
+        const SmRef C = pick(op == 0, mZ, pick(op == 1, mQ, pick(op == 2, mRZ, mR)));
+        sm_product<4>(L, rt, D, C, op == 0 ? c : 1.0f, op == 0 ? b : a, r0, c0, k, lane);
       }
     }
-    out_q = true;
+    mS = mQ;
   }
 
   // ---- S (row-major 128 x 128) to the workspace
   uint16_t* S = d.S[args.so];
   for (int i = threadIdx.x; i < kSm * kSm / 8; i += blockDim.x) {
     const int r = i >> 4, c = i & 15;
-    const SmMat out{out_q ? Q.h0 : Z.h0, out_q ? Q.h1 : Z.h1};
-    glb_store16(S + r * kSm + 8 * c, lds_load16(sm_at(out, r >> 6, r & 63, c)));
+    glb_store16(S + r * kSm + 8 * c, *sm_ref_ptr<const u32x4>(sm_ref_at(mS, r, 8 * c)));
   }
 }
 
@@ -1188,7 +1274,9 @@ __global__ __launch_bounds__(kSmApplyThreads, 1) void pm_small_apply_kernel(Gemm
   int gfin = -1;
   // adds the waiting unit (in tile gt) to R and, at a matrix's end, writes R
   // to its S[sc]
-  auto gram_catch_up = [&](const char* gt) {
+  // (always inlined, like unit below: called, their captures would live in
+  // scratch memory)
+  auto gram_catch_up = [&](const char* gt) __attribute__((always_inline)) {
     if (!gpend) return;
     sm_gram_acc(gt, gacc, gr0, gc0, lane);
     if (gfin >= 0) {
@@ -1214,7 +1302,8 @@ __global__ __launch_bounds__(kSmApplyThreads, 1) void pm_small_apply_kernel(Gemm
   // lets the compiler see that they are not the copies' targets; through a
   // pointer chosen at run time it would wait for every copy in flight before
   // touching them.
-  auto unit = [&](char* xs, const char* ps, char* nxs, char* nps, int u, char* gt, const char* gp) {
+  auto unit = [&](char* xs, const char* ps, char* nxs, char* nps, int u, char* gt,
+                  const char* gp) __attribute__((always_inline)) {
     wait_unit<C>(u - u0);
     if constexpr (!kFinal) wait_lgkmcnt<0>();  // this wave's X' tile writes of unit u-1 are done
     block_barrier();  // every wave's copies of u have landed; every wave is done with unit u-1
