@@ -1666,11 +1666,25 @@ __global__ __launch_bounds__(kThreads) void pm_qinit_kernel(const MatDesc* descs
 // ============================================================ elementwise
 // Bound by HBM. A block moves kEwBlock consecutive elements: every thread
 // kEwVecs runs of 4 (16-byte vectors of fp32, 8-byte ones of bf16, lanes
-// consecutive), all of its loads issued before its stores; the last block
-// element by element past n. (A bf16 5120 x 4096 gradient's momentum 47 -> 37
-// us, its param step 38 -> 19, against one element a thread and iteration.)
+// consecutive), all of its loads issued before its stores; the last block the
+// runs that n leaves it, then up to 3 elements. (A bf16 5120 x 4096 gradient's
+// momentum 47 -> 37 us, its param step 38 -> 19, against one element a thread
+// and iteration.)
 constexpr int kEwVecs = 4;
 constexpr int kEwBlock = kThreads * 4 * kEwVecs;
+
+template <bool W>
+struct EwWhole {
+  static constexpr bool value = W;
+};
+// The thread's run k of its block; of a last block with count > 0 runs, one
+// past them stands for the last (loaded, not stored: a branch a load would make
+// each wait for its own).
+template <bool WHOLE>
+__device__ __forceinline__ int ew_run(int k, int count) {
+  const int v = (int)threadIdx.x + k * kThreads;
+  return WHOLE || v < count ? v : count - 1;
+}
 
 template <bool F32>
 __device__ __forceinline__ f32x4 ew_load(const void* p, int64_t i) {
@@ -1701,17 +1715,18 @@ __global__ __launch_bounds__(kThreads) void pm_momentum_kernel(void* buf, const 
     return nesterov ? omu * g + mu * m : m;
   };
   const int64_t base = (int64_t)blockIdx.x * kEwBlock;
-  if (base + kEwBlock <= n) {
+  auto runs = [&](auto whole, int count) __attribute__((always_inline)) {
     f32x4 g[kEwVecs], m[kEwVecs];
 #pragma unroll
     for (int k = 0; k < kEwVecs; ++k) {
-      const int64_t i = base + 4 * (threadIdx.x + k * kThreads);
+      const int64_t i = base + 4 * ew_run<whole.value>(k, count);
       g[k] = ew_load<G32>(grad, i);
       m[k] = ew_load<B32>(buf, i);
     }
 #pragma unroll
     for (int k = 0; k < kEwVecs; ++k) {
       const int64_t i = base + 4 * (threadIdx.x + k * kThreads);
+      if (!whole.value && (int)threadIdx.x + k * kThreads >= count) return;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         float me = m[k][e];
@@ -1721,9 +1736,11 @@ __global__ __launch_bounds__(kThreads) void pm_momentum_kernel(void* buf, const 
       ew_store<B32>(buf, i, m[k]);
       ew_store<U32>(upd, i, g[k]);
     }
-    return;
-  }
-  for (int64_t i = base + threadIdx.x; i < n; i += kThreads) {
+  };
+  if (base + kEwBlock <= n) return runs(EwWhole<true>{}, 0);
+  if (n - base >= 4) runs(EwWhole<false>{}, (int)(n - base) / 4);
+  const int64_t i = (n & ~(int64_t)3) + threadIdx.x;
+  if (i < n) {
     const float g = load_elem(grad, G32 ? DT_F32 : DT_BF16, i);
     float m = load_elem(buf, B32 ? DT_F32 : DT_BF16, i);
     const float u = step(g, m);
@@ -1745,23 +1762,26 @@ __global__ __launch_bounds__(kThreads) void pm_step_kernel(void* param, const vo
     neg = -(lr * adj);
   }
   const int64_t base = (int64_t)blockIdx.x * kEwBlock;
-  if (base + kEwBlock <= n) {
+  auto runs = [&](auto whole, int count) __attribute__((always_inline)) {
     f32x4 p[kEwVecs], u[kEwVecs];
 #pragma unroll
     for (int k = 0; k < kEwVecs; ++k) {
-      const int64_t i = base + 4 * (threadIdx.x + k * kThreads);
+      const int64_t i = base + 4 * ew_run<whole.value>(k, count);
       p[k] = ew_load<P32>(param, i);
       u[k] = ew_load<U32>(upd, i);
     }
 #pragma unroll
     for (int k = 0; k < kEwVecs; ++k) {
+      if (!whole.value && (int)threadIdx.x + k * kThreads >= count) return;
 #pragma unroll
       for (int e = 0; e < 4; ++e) p[k][e] = p[k][e] * wdf + u[k][e] * neg;
       ew_store<P32>(param, base + 4 * (threadIdx.x + k * kThreads), p[k]);
     }
-    return;
-  }
-  for (int64_t i = base + threadIdx.x; i < n; i += kThreads) {
+  };
+  if (base + kEwBlock <= n) return runs(EwWhole<true>{}, 0);
+  if (n - base >= 4) runs(EwWhole<false>{}, (int)(n - base) / 4);
+  const int64_t i = (n & ~(int64_t)3) + threadIdx.x;
+  if (i < n) {
     const float p = load_elem(param, P32 ? DT_F32 : DT_BF16, i);
     const float u = load_elem(upd, U32 ? DT_F32 : DT_BF16, i);
     store_elem(param, P32 ? DT_F32 : DT_BF16, i, p * wdf + u * neg);
