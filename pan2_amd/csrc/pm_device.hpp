@@ -4,7 +4,8 @@
 // launches, each walking every matrix of the group:
 //   pm_prologue_kernel   momentum update + bf16 X write + per-tile Σx²
 //   pm_norm_kernel       per-matrix 1/‖X‖ and 1/‖X‖²
-//   pm_ns_gemm_kernel    x ns_steps x {GRAM, POLY, UPDATE|FINAL}
+//   pm_ns_gemm_kernel    x ns_steps x {GRAM, POLY, UPDATE|FINAL}, a stage as
+//                        pm_tile_gemm_kernel where 256-tiles leave CUs idle
 // The GEMM kernel is one bf16 MFMA (v_mfma_f32_16x16x32_bf16) tile engine
 // with four epilogues; its operands are read K-contiguous from LDS, except X
 // in C = S·X and C = Xᵀ·S, which is read transposed from LDS.
@@ -47,13 +48,13 @@ struct MatDesc {
   int32_t p_dt, g_dt, m_dt;
   int32_t trans;      // rows > cols: X = uᵀ so the short side is contracted
   int32_t M, N;       // short and long side
-  int32_t Mp, Np;     // padded to kTile (padding is zero and stays zero)
+  int32_t Mp, Np;     // padded to kTile (zero, and stays so, where 256-tiles read it)
   float adj_ratio;    // device-lr path: adjusted_lr = lr * adj_ratio
   float neg_lr_host;  // host-lr path: -(lr * adj_ratio), rounded once
   // workspace buffers
   // X and S are in the panel layout of ws_off for large matrices; a small
   // matrix (Mp = 128) keeps X in the layout of sm_x_off
-  uint16_t* X[2];     // bf16 Mp x Np (ld Np), ping-pong
+  uint16_t* X[2];     // bf16 Mp x Np (ld Np), ping-pong; one buffer twice for a small matrix
   // bf16 Mp x Mp work matrices. Standard form: S[0] = A = X Xᵀ,
   // S[1] = B = b A + c A². Gram form: S[0] = R, S[1] = Z, S[2] = R Z + a R,
   // S[3], S[4] = Q (ping-pong). Unused entries are null.
