@@ -374,3 +374,33 @@ def test_factory_adamw_runs_on_libpanmuon_and_round_trips_state():
         assert torch.equal(pa, pb)
         moved += int(not torch.equal(pa, ps))
     assert moved == 4  # the AdamW params (two biases, the LayerNorm weight and bias) moved; not the Muon weights
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("off", [1, 2, 5])
+def test_tensors_off_16_bytes_equal_aligned_ones(dt, off):
+    """Tensors that start off elements into their allocation give the bits of
+    aligned ones, and nothing around them changes."""
+    print(f"adam off {off} {dt}", flush=True)
+    sizes = [1, 7, 8, 9, 8191, 8192, 8193, 100003]
+    kw = dict(lr=2e-3, beta1=0.9, beta2=0.95, eps=1e-8, weight_decay=0.05, amsgrad=True, maximize=False,
+              decoupled=True)
+    results = []
+    for o in (0, off):
+        bufs, views = [], []
+        for k in range(5):  # params, grads, exp_avgs, exp_avg_sqs, max_exp_avg_sqs
+            row = []
+            for i, n in enumerate(sizes):
+                buf = torch.full((n + 16,), 3.0, dtype=DT[dt], device=DEV)
+                x = as_dtype(np.abs(rnd(n, 10 * k + i, 0.1)) if k > 2 else rnd(n, 10 * k + i, 0.1), dt)
+                buf[o:o + n] = dev(x, dt)
+                bufs.append((buf, n))
+                row.append(buf[o:o + n])
+            views.append(row)
+        steps = [torch.full((), 4.0, device=DEV) for _ in sizes]
+        _lib.adam_step(*views, steps, **kw)
+        for buf, n in bufs:
+            assert bool((buf[:o] == 3.0).all()) and bool((buf[o + n:] == 3.0).all())
+        results.append([t.clone() for row in views for t in row])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)

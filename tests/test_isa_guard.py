@@ -136,3 +136,13 @@ def test_small_kernels_keep_lds_in_lds(asm):
     body = kernels[gram_apply[0]]
     assert not re.findall(r"^\s*flat_", body, flags=re.M), gram_apply[0]
     assert "ds_write_b64" in body and "ds_read_b128" in body, gram_apply[0]
+
+
+def test_adam_kernel_has_one_element_loop_per_access(asm):
+    """Each of the Adam kernel's accesses is its vectors or one unrolled loop
+    over single elements: 3725 instructions. A second copy of that loop behind
+    another condition, as for unaligned tensors alone, made it 5018."""
+    m = re.search(r"^_ZN2pm14pm_adam_kernel\w+:.*$", asm, flags=re.M)
+    body = asm[m.end():]
+    n = len(re.findall(r"^\t[a-z]", body[:body.index(".Lfunc_end")], flags=re.M))
+    assert n < 4200, n
