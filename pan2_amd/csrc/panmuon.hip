@@ -1016,9 +1016,23 @@ int collect_ns(const pm_ns_matrix* mats, int n, int form, std::vector<Item>& ite
   return PM_OK;
 }
 
-// The elementwise kernels' launches, by the tensors' dtypes; kernels' grids
-// stay below 2^31 blocks for any tensor that fits the GPU.
-int64_t ew_blocks(int64_t n) { return (n + kEwBlock - 1) / kEwBlock; }
+// The elementwise kernels' launches, by the tensors' dtypes. A launch holds
+// fewer than 2^32 threads, so a longer tensor goes in several.
+constexpr int64_t kEwLaunch = (int64_t)kEwBlock << 23;  // elements of a launch: whole blocks
+static_assert(kEwLaunch / kEwBlock * kThreads < (1ll << 32), "threads of a launch");
+
+// Calls launch(offset, elements, grid) for the launches that cover n elements.
+template <class F>
+void ew_launches(int64_t n, F launch) {
+  for (int64_t off = 0; off < n; off += kEwLaunch) {
+    const int64_t count = std::min(n - off, kEwLaunch);
+    launch(off, count, dim3((uint32_t)((count + kEwBlock - 1) / kEwBlock)));
+  }
+}
+
+// element off of an f32 or bf16 tensor
+void* ew_at(void* base, bool f32, int64_t off) { return (char*)base + off * (f32 ? 4 : 2); }
+const void* ew_at(const void* base, bool f32, int64_t off) { return (const char*)base + off * (f32 ? 4 : 2); }
 
 template <bool B32, bool G32>
 void launch_momentum(bool u32, dim3 grid, hipStream_t stream, void* buf, const void* grad, void* update, int64_t n,
@@ -1189,14 +1203,16 @@ int pm_momentum_nesterov(void* buf, int32_t buf_dtype, const void* grad, int32_t
   if (!buf || !grad || !update) return fail(PM_EINVAL, "NULL tensor pointer");
   if (!valid_dtype(buf_dtype) || !valid_dtype(grad_dtype) || !valid_dtype(update_dtype))
     return fail(PM_EDTYPE, "dtypes must be f32 or bf16");
-  if (ew_blocks(n) > INT32_MAX) return fail(PM_EINVAL, "too many elements in one call");
-  const dim3 grid((uint32_t)ew_blocks(n));
   const bool b32 = buf_dtype == PM_DTYPE_F32, g32 = grad_dtype == PM_DTYPE_F32, u32 = update_dtype == PM_DTYPE_F32;
-  const hipStream_t s = (hipStream_t)stream;
-  if (b32 && g32) launch_momentum<true, true>(u32, grid, s, buf, grad, update, n, momentum, nesterov);
-  else if (b32) launch_momentum<true, false>(u32, grid, s, buf, grad, update, n, momentum, nesterov);
-  else if (g32) launch_momentum<false, true>(u32, grid, s, buf, grad, update, n, momentum, nesterov);
-  else launch_momentum<false, false>(u32, grid, s, buf, grad, update, n, momentum, nesterov);
+  ew_launches(n, [&](int64_t off, int64_t count, dim3 grid) {
+    const hipStream_t s = (hipStream_t)stream;
+    void *b = ew_at(buf, b32, off), *u = ew_at(update, u32, off);
+    const void* g = ew_at(grad, g32, off);
+    if (b32 && g32) launch_momentum<true, true>(u32, grid, s, b, g, u, count, momentum, nesterov);
+    else if (b32) launch_momentum<true, false>(u32, grid, s, b, g, u, count, momentum, nesterov);
+    else if (g32) launch_momentum<false, true>(u32, grid, s, b, g, u, count, momentum, nesterov);
+    else launch_momentum<false, false>(u32, grid, s, b, g, u, count, momentum, nesterov);
+  });
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? PM_OK : hip_fail(e, "momentum launch");
 }
@@ -1210,13 +1226,15 @@ int pm_step_param(void* param, int32_t param_dtype, const void* update, int32_t 
   if (!valid_dtype(param_dtype) || !valid_dtype(update_dtype)) return fail(PM_EDTYPE, "dtypes must be f32 or bf16");
   const float wdf = (float)(1.0 - lr_host * (double)weight_decay);
   const float neg = (float)(-(lr_host * adj_ratio));
-  if (ew_blocks(n) > INT32_MAX) return fail(PM_EINVAL, "too many elements in one call");
-  const dim3 grid((uint32_t)ew_blocks(n));
-  const bool u32 = update_dtype == PM_DTYPE_F32;
-  if (param_dtype == PM_DTYPE_F32)
-    launch_step<true>(u32, grid, (hipStream_t)stream, param, update, n, lr_dev, weight_decay, (float)adj_ratio, wdf, neg);
-  else
-    launch_step<false>(u32, grid, (hipStream_t)stream, param, update, n, lr_dev, weight_decay, (float)adj_ratio, wdf, neg);
+  const bool p32 = param_dtype == PM_DTYPE_F32, u32 = update_dtype == PM_DTYPE_F32;
+  ew_launches(n, [&](int64_t off, int64_t count, dim3 grid) {
+    const hipStream_t s = (hipStream_t)stream;
+    void* p = ew_at(param, p32, off);
+    const void* u = ew_at(update, u32, off);
+    const float wd = weight_decay, adj = (float)adj_ratio;
+    if (p32) launch_step<true>(u32, grid, s, p, u, count, lr_dev, wd, adj, wdf, neg);
+    else launch_step<false>(u32, grid, s, p, u, count, lr_dev, wd, adj, wdf, neg);
+  });
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? PM_OK : hip_fail(e, "step launch");
 }

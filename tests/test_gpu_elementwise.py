@@ -55,3 +55,19 @@ def test_step(n, dtypes):
     want = muon_ref.step_param(p0.float().cpu().numpy(), u.float().cpu().numpy(), 0.02, 0.01, 1.5)
     assert torch.equal(p.cpu(), torch.from_numpy(np.asarray(want, dtype=np.float32)).to(dtypes[0]))
     assert torch.equal(pb[:off], was[:off]) and torch.equal(pb[off + n:], was[off + n:])
+
+
+def test_step_of_more_elements_than_one_launch_holds():
+    """2^36 elements are 2^24 blocks, 2^32 threads: more than a launch may
+    hold. The tensor is its own update, so that one of 128 GiB does."""
+    n = (1 << 36) + 4099
+    if torch.cuda.mem_get_info()[0] < 2 * n + (8 << 30):
+        pytest.skip("needs 136 GiB of free GPU memory")
+    p = torch.ones(n, dtype=B, device=DEV)
+    try:
+        _lib.step_param_inplace(p, p, 0.5, 0.0, 1.0)  # p - 0.5 p, exact
+        for i in range(0, n, 1 << 30):
+            assert bool((p[i:i + (1 << 30)] == 0.5).all()), i
+    finally:
+        del p
+        torch.cuda.empty_cache()
