@@ -76,6 +76,11 @@ struct Plan {
 // needs one, the S its core launch hands to its apply launch.
 int square_bufs(int form, bool small) { return small ? 1 : form == NS_GRAM ? 5 : 2; }
 
+// Mp x Np buffers per matrix: X and X', or one for a small matrix, whose apply
+// updates X in place (each unit of X' depends on the same unit of X only,
+// which its block has read into LDS).
+int x_bufs(bool small) { return small ? 1 : 2; }
+
 Plan make_plan(int64_t rows, int64_t cols, int form) {
   Plan p{};
   p.rows = (int32_t)rows;
@@ -89,11 +94,11 @@ Plan make_plan(int64_t rows, int64_t cols, int form) {
   const size_t x = align_up((size_t)p.Mp * p.Np * 2);
   const size_t a = align_up((size_t)p.Mp * p.Mp * 2);
   const size_t part = align_up((size_t)(p.Mp / kProTile) * (p.Np / kProTile) * 4);  // (covers every run count)
-  // X ping-pong, the square work matrices, the prologue partials; split_call
-  // adds the K-split partials
+  // X, the square work matrices, the prologue partials; split_call adds the
+  // K-split partials
   p.ks_gram = p.ks_symm = p.ks_full = 1;
   p.kpart = 0;
-  p.ws = 2 * x + (size_t)square_bufs(form, p.small) * a + part + kAlign;
+  p.ws = (size_t)x_bufs(p.small) * x + (size_t)square_bufs(form, p.small) * a + part + kAlign;
   const double M = p.M, N = p.N;
   p.flops = M * (M + 1) * N + M * M * (M + 1) + 2 * M * M * N;
   return p;
@@ -785,10 +790,8 @@ int run_group(Item* items, int count, int group, const pm_hparams* hp, int mode,
     d.M = p.M; d.N = p.N; d.Mp = p.Mp; d.Np = p.Np;
     const size_t x = align_up((size_t)p.Mp * p.Np * 2);
     const size_t a = align_up((size_t)p.Mp * p.Mp * 2);
-    d.X[0] = (uint16_t*)cursor; cursor += x;
-    // a small matrix's apply updates X in place (each unit of X' depends on the
-    // same unit of X only, which its block has read into LDS)
-    d.X[1] = small ? d.X[0] : (uint16_t*)cursor; cursor += x;
+    for (int b = 0; b < 2; ++b) d.X[b] = (uint16_t*)(cursor + (b < x_bufs(p.small) ? b * x : 0));
+    cursor += x_bufs(p.small) * x;
     for (int b = 0; b < kSquareBufs; ++b) {
       d.S[b] = b < square_bufs(form, p.small) ? (uint16_t*)cursor : nullptr;
       if (b < square_bufs(form, p.small)) cursor += a;

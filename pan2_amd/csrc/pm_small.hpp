@@ -1446,7 +1446,7 @@ __global__ __launch_bounds__(kSmApplyThreads, 1) void pm_small_apply_kernel(Gemm
   };
 
   // slot S holds unit u0 + S (mod kRing); unit S releases slot S - 1 to the copy walk
-  static_assert(!GRAM || kRing % 2 == 0, "X' tiles alternate with the ring slots");
+  static_assert(kFinal || kRing % 2 == 0, "X' tiles alternate with the ring slots");
 #define PM_SM_UNIT(S)                                                                                 \
   unit(sl.x[S], sl.p[(S) & 3], sl.x[((S) + kRing - 1) % kRing], sl.p[(((S) + kRing - 1) % kRing) & 3], u + (S), \
        ((S) & 1) ? gt1 : gt0, ((S) & 1) ? gt0 : gt1)

@@ -333,6 +333,18 @@ def test_gram_form_workspace_sizing(lib):
     assert gram - std <= 3 * M * M * 2 + (64 << 10)  # plus a larger launch table
 
 
+@pytest.mark.parametrize("form", ["standard", "gram"])
+def test_small_matrix_workspace_holds_one_x(lib, form):
+    """A small matrix's X is updated in place: one 128 x Np buffer and one
+    128 x 128, beside the prologue's partials and the table."""
+    hp = hparams(ns_form=form)
+    ws = lambda n: lib.pm_workspace_bytes(arr(*[mat(128, 4096)] * n), n, ctypes.byref(hp))  # noqa: E731
+    x, sq = 128 * 4096 * 2, 128 * 128 * 2
+    part = 2 * (4096 // 64) * 4 + 256
+    each = (ws(64) - ws(32)) / 32
+    assert x + sq + part <= each <= x + sq + part + 1024  # and its table entries
+
+
 def test_ns_workspace_matches_step_workspace(lib):
     m = _lib.PmNsMatrix()
     m.in_, m.out = FAKE, FAKE
