@@ -437,12 +437,12 @@ struct Launcher {
   // when some matrix splits this stage, the GEMM over their chunk items
   // (fp32 partials) and the reduce over their tiles. The stage's FLOPs go
   // with its first launch.
-  template <int STAGE, int T, int NW, int RING>
+  template <int STAGE, int T, int NW>
   int tile_launch(GemmArgs a, const Stage& st, int kind, int it, double flops, const char* what) {
     if (st.tiles_total > 0) {
       a.prefix = st.tiles;
       a.total = st.tiles_total;
-      hipLaunchKernelGGL((pm_tile_gemm_kernel<STAGE, T, NW, RING, false>), dim3(st.persistent ? gemm_grid(a.total) : a.total), dim3(64 * NW), 0, stream, a);
+      hipLaunchKernelGGL((pm_tile_gemm_kernel<STAGE, T, NW, false>), dim3(st.persistent ? gemm_grid(a.total) : a.total), dim3(64 * NW), 0, stream, a);
       timing_mark(stream, kind, group, it, count, flops, 0.0);
       flops = 0.0;
       if (int rc = check(what)) return rc;
@@ -450,7 +450,7 @@ struct Launcher {
     if (st.items_total == 0) return PM_OK;
     a.prefix = st.items;
     a.total = st.items_total;
-    hipLaunchKernelGGL((pm_tile_gemm_kernel<STAGE, T, NW, RING, true>), dim3(st.persistent ? gemm_grid(a.total) : a.total), dim3(64 * NW), 0, stream, a);
+    hipLaunchKernelGGL((pm_tile_gemm_kernel<STAGE, T, NW, true>), dim3(st.persistent ? gemm_grid(a.total) : a.total), dim3(64 * NW), 0, stream, a);
     timing_mark(stream, kind, group, it, count, flops, 0.0);
     if (int rc = check(what)) return rc;
     a.prefix = st.split;
@@ -461,8 +461,8 @@ struct Launcher {
   }
   template <int STAGE, int PDT>
   int stage_launch(GemmArgs a, const Stage& st, int kind, int it, double flops, const char* what) {
-    if (st.edge == 64) return tile_launch<STAGE, 64, 4, 4>(a, st, kind, it, flops, what);
-    if (st.edge == 128) return tile_launch<STAGE, 128, 8, 4>(a, st, kind, it, flops, what);
+    if (st.edge == 64) return tile_launch<STAGE, 64, 4>(a, st, kind, it, flops, what);
+    if (st.edge == 128) return tile_launch<STAGE, 128, 8>(a, st, kind, it, flops, what);
     if (st.tiles_total > 0) {
       a.prefix = st.tiles;
       a.total = st.tiles_total;

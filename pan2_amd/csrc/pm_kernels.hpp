@@ -1644,6 +1644,7 @@ __global__ __launch_bounds__(64) void pm_ns_reduce_kernel(GemmArgs args) {
 __global__ __launch_bounds__(kThreads) void pm_qinit_kernel(const MatDesc* descs, int32_t first, int32_t sz,
                                                             int32_t sq, float a) {
 #pragma clang fp contract(off)
+  static_assert((kWsLayout & kTiledS) != 0, "a block's half unit is consecutive in the panel layout only");
   const MatDesc& d = descs[first + blockIdx.y];
   const int units = d.Mp / 64, x = blockIdx.x >> 1;  // unit x of the matrix: panel x / units, columns 64·(x % units)
   if (x >= d.Mp / kTile * units) return;

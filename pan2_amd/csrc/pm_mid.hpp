@@ -29,11 +29,13 @@
 namespace pm {
 
 constexpr int kMtRun = 16;  // consecutive items an XCD takes at once (xcd_runs)
+constexpr int kMtRing = 4;  // LDS slots, each one unit of both operands
+static_assert(kWsLayout == (kTiledX | kTiledS), "the copies and epilogues assume panel layouts of X and S");
 
 // Blocks of NW waves in a 2 x NW/2 grid over the T x T tile.
 template <int T, int NW>
 struct MtTile {
-  static_assert((T == 64 && NW == 4) || (T == 128 && (NW == 4 || NW == 8)), "tile edge and waves");
+  static_assert((T == 64 && NW == 4) || (T == 128 && NW == 8), "tile edge and waves");
   static constexpr int kOp = T * 128;          // one operand of one unit: T rows (or columns) x 64 k
   static constexpr int kRows = T / 2;          // a wave's rows and columns of the tile
   static constexpr int kCols = 2 * T / NW;
@@ -192,32 +194,31 @@ __device__ __forceinline__ void mt_wait(int n) {
   else wait_vmcnt<0>();
 }
 
-template <int RING>
 struct MtRing {
-  char* a[RING];
-  char* b[RING];
+  char* a[kMtRing];
+  char* b[kMtRing];
 };
 
-// Unit u, whose fragments are in f[S % 2], from a ring of RING slots (unit u in
-// slot S = (u - u0) % RING): once every wave's copies of u + 1 have landed and
-// every wave has read u, refill u's slot with unit u + RING, read u + 1's
+// Unit u, whose fragments are in f[S % 2], from the ring (unit u in slot
+// S = (u - u0) % kMtRing): once every wave's copies of u + 1 have landed and
+// every wave has read u, refill u's slot with unit u + kMtRing, read u + 1's
 // fragments, and run u's MFMAs behind those reads.
-// STEADY: units u + 1 .. u + RING exist, so nothing is conditional (a
+// STEADY: units u + 1 .. u + kMtRing exist, so nothing is conditional (a
 // conditional copy or wait would make the compiler, which tracks copies into
 // LDS along every path, drain them all before a read).
-template <int T, int NW, bool TR, int RING, int S, bool STEADY>
-__device__ __forceinline__ void mt_step(const MtRing<RING>& ring, const MtCopy<T, NW, TR>& copy, int u, int u1,
+template <int T, int NW, bool TR, int S, bool STEADY>
+__device__ __forceinline__ void mt_step(const MtRing& ring, const MtCopy<T, NW, TR>& copy, int u, int u1,
                                         MtFrags<T, NW> (&f)[2],
                                         f32x4 (&acc)[MtTile<T, NW>::kQi][MtTile<T, NW>::kQj], int lane) {
   typedef MtTile<T, NW> C;
   if (STEADY || u + 1 < u1) {
-    if (STEADY) wait_vmcnt<(RING - 2) * 2 * C::kCopies>();
-    else mt_wait<T, NW>(imin(RING - 2, u1 - 2 - u));
+    if (STEADY) wait_vmcnt<(kMtRing - 2) * 2 * C::kCopies>();
+    else mt_wait<T, NW>(imin(kMtRing - 2, u1 - 2 - u));
     wait_lgkmcnt<0>();
     block_barrier();
-    mt_read<T, NW, TR>(ring.a[(S + 1) % RING], ring.b[(S + 1) % RING], f[(S + 1) & 1], copy.wave, lane);
+    mt_read<T, NW, TR>(ring.a[(S + 1) % kMtRing], ring.b[(S + 1) % kMtRing], f[(S + 1) & 1], copy.wave, lane);
     __builtin_amdgcn_sched_barrier(0);
-    if (STEADY || u + RING < u1) copy(ring.a[S], ring.b[S], u + RING);
+    if (STEADY || u + kMtRing < u1) copy(ring.a[S], ring.b[S], u + kMtRing);
     __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
@@ -447,15 +448,14 @@ __device__ __forceinline__ f32x4* mt_partial(float* kpart, int tiles, int tile, 
 // tile, or (SPLIT) a chunk of a tile's K range. Block b takes items b,
 // b + gridDim, ...; with fewer blocks than items (persistent) an item's first
 // units are requested before the previous item's epilogue.
-template <int STAGE, int T, int NW, int RING, bool SPLIT>
+template <int STAGE, int T, int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW, T == 64 ? 2 : 1) void pm_tile_gemm_kernel(GemmArgs args) {
-  static_assert(RING == 4, "ring depth");
   typedef MtTile<T, NW> C;
   constexpr int kOp = C::kOp;
   constexpr bool TR = STAGE == ST_UPDATE || STAGE == ST_FINAL;
   __shared__ __attribute__((aligned(1024))) char a0[kOp], b0[kOp], a1[kOp], b1[kOp], a2[kOp], b2[kOp], a3[kOp], b3[kOp];
   __shared__ __attribute__((aligned(1024))) char tile_lds[SPLIT ? 16 : 64 * T * 4];
-  MtRing<RING> ring;  // (set member by member: an aggregate initialiser of LDS addresses does not compile)
+  MtRing ring;  // (set member by member: an aggregate initialiser of LDS addresses does not compile)
   ring.a[0] = a0; ring.b[0] = b0; ring.a[1] = a1; ring.b[1] = b1;
   ring.a[2] = a2; ring.b[2] = b2; ring.a[3] = a3; ring.b[3] = b3;
   typedef const __attribute__((address_space(4))) MatDesc* DescPtr;
@@ -475,7 +475,7 @@ __global__ __launch_bounds__(64 * NW, T == 64 ? 2 : 1) void pm_tile_gemm_kernel(
   auto start = [&](const MtJob& j) {
     const MtCopy<T, NW, TR> copy(j, wave, lane);
 #pragma unroll
-    for (int i = 0; i < RING; ++i) copy(ring.a[i], ring.b[i], imin(j.u0 + i, j.u1 - 1));
+    for (int i = 0; i < kMtRing; ++i) copy(ring.a[i], ring.b[i], imin(j.u0 + i, j.u1 - 1));
   };
   MtJob job = decode(b);
   start(job);
@@ -493,19 +493,19 @@ __global__ __launch_bounds__(64 * NW, T == 64 ? 2 : 1) void pm_tile_gemm_kernel(
     wait_lgkmcnt<0>();
     block_barrier();
     mt_read<T, NW, TR>(ring.a[0], ring.b[0], f[0], wave, lane);
-    for (; u + 2 * RING <= u1; u += RING) {
-      mt_step<T, NW, TR, RING, 0, true>(ring, copy, u, u1, f, acc, lane);
-      mt_step<T, NW, TR, RING, 1, true>(ring, copy, u + 1, u1, f, acc, lane);
-      mt_step<T, NW, TR, RING, 2, true>(ring, copy, u + 2, u1, f, acc, lane);
-      mt_step<T, NW, TR, RING, 3, true>(ring, copy, u + 3, u1, f, acc, lane);
+    for (; u + 2 * kMtRing <= u1; u += kMtRing) {
+      mt_step<T, NW, TR, 0, true>(ring, copy, u, u1, f, acc, lane);
+      mt_step<T, NW, TR, 1, true>(ring, copy, u + 1, u1, f, acc, lane);
+      mt_step<T, NW, TR, 2, true>(ring, copy, u + 2, u1, f, acc, lane);
+      mt_step<T, NW, TR, 3, true>(ring, copy, u + 3, u1, f, acc, lane);
     }
-    // at most 2·RING - 1 units are left
+    // at most 2·kMtRing - 1 units are left
 #pragma unroll 1
-    for (; u < u1; u += RING) {
-      mt_step<T, NW, TR, RING, 0, false>(ring, copy, u, u1, f, acc, lane);
-      if (u + 1 < u1) mt_step<T, NW, TR, RING, 1, false>(ring, copy, u + 1, u1, f, acc, lane);
-      if (u + 2 < u1) mt_step<T, NW, TR, RING, 2, false>(ring, copy, u + 2, u1, f, acc, lane);
-      if (u + 3 < u1) mt_step<T, NW, TR, RING, 3, false>(ring, copy, u + 3, u1, f, acc, lane);
+    for (; u < u1; u += kMtRing) {
+      mt_step<T, NW, TR, 0, false>(ring, copy, u, u1, f, acc, lane);
+      if (u + 1 < u1) mt_step<T, NW, TR, 1, false>(ring, copy, u + 1, u1, f, acc, lane);
+      if (u + 2 < u1) mt_step<T, NW, TR, 2, false>(ring, copy, u + 2, u1, f, acc, lane);
+      if (u + 3 < u1) mt_step<T, NW, TR, 3, false>(ring, copy, u + 3, u1, f, acc, lane);
     }
     wait_lgkmcnt<0>();
     block_barrier();  // every wave has read the last unit
