@@ -328,7 +328,7 @@ typedef struct pm_launch_time {
   double flops;        /* algorithmic FLOPs (GEMM launches) */
   double bytes;        /* algorithmic HBM bytes (prologue) */
   float ms;            /* event-measured duration */
-  float reserved;
+  int32_t tile;        /* GEMM launches and their reduces: tile edge (256, 128 or 64), else 0 */
 } pm_launch_time;
 
 int pm_timing_enable(int on);

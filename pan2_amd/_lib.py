@@ -149,7 +149,7 @@ class PmLaunchTime(ctypes.Structure):
         ("flops", ctypes.c_double),
         ("bytes", ctypes.c_double),
         ("ms", ctypes.c_float),
-        ("reserved", ctypes.c_float),
+        ("tile", ctypes.c_int32),
     ]
 
 
@@ -688,4 +688,4 @@ def timing_read(max_records: int = 1 << 16) -> list[dict]:
     if n < 0:
         check(n, "pm_timing_read")
     return [dict(kind=KERNEL_KINDS[r.kind], group=r.group, iteration=r.iteration, n_matrices=r.n_matrices,
-                 flops=r.flops, bytes=r.bytes, ms=r.ms) for r in buf[:n]]
+                 flops=r.flops, bytes=r.bytes, ms=r.ms, tile=r.tile) for r in buf[:n]]

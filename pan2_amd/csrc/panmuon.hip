@@ -383,7 +383,8 @@ void timing_begin(hipStream_t stream) {
 }
 
 // Records the end of the launch just enqueued on `stream`.
-void timing_mark(hipStream_t stream, int kind, int group, int iteration, int nmat, double flops, double bytes) {
+void timing_mark(hipStream_t stream, int kind, int group, int iteration, int nmat, double flops, double bytes,
+                 int tile = 0) {
   if (!g_timing.on.load(std::memory_order_relaxed)) return;
   std::lock_guard<std::mutex> lock(g_timing.mu);
   if (!g_timing.last || g_timing.last_stream != stream) return;
@@ -400,6 +401,7 @@ void timing_mark(hipStream_t stream, int kind, int group, int iteration, int nma
   r.info.n_matrices = nmat;
   r.info.flops = flops;
   r.info.bytes = bytes;
+  r.info.tile = tile;
   r.begin = g_timing.last;
   r.end = e;
   g_timing.recs.push_back(r);
@@ -443,7 +445,7 @@ struct Launcher {
       a.prefix = st.tiles;
       a.total = st.tiles_total;
       hipLaunchKernelGGL((pm_tile_gemm_kernel<STAGE, T, NW, false>), dim3(st.persistent ? gemm_grid(a.total) : a.total), dim3(64 * NW), 0, stream, a);
-      timing_mark(stream, kind, group, it, count, flops, 0.0);
+      timing_mark(stream, kind, group, it, count, flops, 0.0, T);
       flops = 0.0;
       if (int rc = check(what)) return rc;
     }
@@ -451,12 +453,12 @@ struct Launcher {
     a.prefix = st.items;
     a.total = st.items_total;
     hipLaunchKernelGGL((pm_tile_gemm_kernel<STAGE, T, NW, true>), dim3(st.persistent ? gemm_grid(a.total) : a.total), dim3(64 * NW), 0, stream, a);
-    timing_mark(stream, kind, group, it, count, flops, 0.0);
+    timing_mark(stream, kind, group, it, count, flops, 0.0, T);
     if (int rc = check(what)) return rc;
     a.prefix = st.split;
     a.total = st.split_total;
     hipLaunchKernelGGL((pm_tile_reduce_kernel<STAGE, T, NW>), dim3(a.total), dim3(64 * NW), 0, stream, a);
-    timing_mark(stream, PM_K_REDUCE, group, it, count, 0.0, 0.0);
+    timing_mark(stream, PM_K_REDUCE, group, it, count, 0.0, 0.0, T);
     return check("K-split reduce launch");
   }
   template <int STAGE, int PDT>
@@ -469,7 +471,7 @@ struct Launcher {
       if (int rc = next_queues(a)) return rc;
       hipLaunchKernelGGL((pm_ns_gemm_kernel<STAGE, PDT, kWsLayout>), dim3(gemm_grid(st.tiles_total)),
                          dim3(kGemmThreads), 0, stream, a);
-      timing_mark(stream, kind, group, it, count, flops, 0.0);
+      timing_mark(stream, kind, group, it, count, flops, 0.0, kTile);
       flops = 0.0;
       if (int rc = check(what)) return rc;
     }
@@ -479,7 +481,7 @@ struct Launcher {
     if (int rc = next_queues(a)) return rc;
     hipLaunchKernelGGL((pm_ns_gemm_kernel<STAGE, PDT, kWsLayout, true>), dim3(gemm_grid(st.items_total)),
                        dim3(kGemmThreads), 0, stream, a);
-    timing_mark(stream, kind, group, it, count, flops, 0.0);
+    timing_mark(stream, kind, group, it, count, flops, 0.0, kTile);
     if (int rc = check(what)) return rc;
     a.prefix = st.split;
     a.total = st.split_total;
@@ -487,7 +489,7 @@ struct Launcher {
     // one single-wave block per (split tile, 128 x 64 sub-tile)
     hipLaunchKernelGGL((pm_ns_reduce_kernel<STAGE, PDT, kWsLayout>), dim3(st.split_total * (kGemmThreads / 64)),
                        dim3(64), 0, stream, a);
-    timing_mark(stream, PM_K_REDUCE, group, it, count, 0.0, 0.0);
+    timing_mark(stream, PM_K_REDUCE, group, it, count, 0.0, 0.0, kTile);
     return check("K-split reduce launch");
   }
   int gram(int cur, bool first, int sc, int it) {

@@ -1,4 +1,4 @@
-"""Static checks of the GEMM kernels' gfx950 assembly (CPU only; hipcc -S).
+"""Static checks of the kernels' gfx950 assembly (CPU only; hipcc -S).
 
 The GEMM engine issues its MFMAs from inline asm with the accumulators tied
 in AGPRs, so the compiler does not know their latency. Three things would
@@ -58,6 +58,26 @@ def reduce_kernels(asm):
     return kernels
 
 
+@pytest.fixture(scope="module")
+def tile_kernels(asm):
+    """The small-tile engine: pm_tile_gemm_kernel and pm_tile_reduce_kernel."""
+    kernels = {}
+    for m in re.finditer(r"^(_ZN2pm\d+pm_tile_(?:gemm|reduce)_kernel\w+):.*$", asm, flags=re.M):
+        body = asm[m.end():]
+        kernels[m.group(1)] = body[:body.index(".Lfunc_end")].split("\n")
+    # GRAM, POLY, UPDATE, FINAL at 64 and 128, unsplit and split, and the reduces
+    assert len(kernels) == 24 and sum("gemm" in k for k in kernels) == 16, sorted(kernels)
+    return kernels
+
+
+def test_tile_kernels_have_no_scratch(tile_kernels):
+    """Their copies are waited for by exact vmcnt counts, which spill traffic
+    would join."""
+    for name, lines in tile_kernels.items():
+        n = sum(1 for ln in lines if "scratch_" in ln)
+        assert n == 0, f"{name}: {n} scratch instructions"
+
+
 def test_reduce_kernels_have_no_scratch(reduce_kernels):
     for name, lines in reduce_kernels.items():
         n = sum(1 for ln in lines if "scratch_" in ln)
@@ -100,11 +120,11 @@ def test_loads_do_not_overwrite_queued_mfma_sources(gemm_kernels):
                 assert not any(dst & src for src in recent), f"{name}: {t}"
 
 
-def test_no_scalar_memory_writes(gemm_kernels):
+def test_no_scalar_memory_writes(gemm_kernels, tile_kernels):
     """Every store and atomic goes through the vector memory path (the tile
     queues' counters included)."""
     bad = re.compile(r"^\s*(s_store|s_buffer_store|s_atomic|s_buffer_atomic|s_scratch_store|s_dcache_wb)")
-    for name, lines in gemm_kernels.items():
+    for name, lines in {**gemm_kernels, **tile_kernels}.items():
         hits = [ln.strip() for ln in lines if bad.match(ln)]
         assert not hits, f"{name}: {hits[:2]}"
 
