@@ -158,6 +158,17 @@ def test_small_kernels_keep_lds_in_lds(asm):
     assert "ds_write_b64" in body and "ds_read_b128" in body, gram_apply[0]
 
 
+def test_prologue_reads_the_extents_once(asm):
+    """rows and cols (bytes 48 and 52 of the descriptor) are read before the
+    loop over a block's runs, by scalar loads: read inside it, behind the loop's
+    stores, they are memory loads that every run's own loads wait for."""
+    m = re.search(r"^_ZN2pm18pm_prologue_kernel\w+:.*$", asm, flags=re.M)
+    body = asm[m.end():]
+    body = body[:body.index(".Lfunc_end")]
+    assert re.search(r"global_load_\w+ .*, s\[\d+:\d+\] offset:32\b", body)  # (the descriptor's g_ld, as it is read there)
+    assert not re.search(r"global_load_\w+ .*, s\[\d+:\d+\] offset:(48|52)\b", body)
+
+
 def test_adam_kernel_has_one_element_loop_per_access(asm):
     """Each of the Adam kernel's accesses is its vectors or one unrolled loop
     over single elements: 3725 instructions. A second copy of that loop behind
