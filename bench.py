@@ -457,7 +457,8 @@ def main() -> int:
                     "avg_launch_ms": round(up_ms / max(1, len(ups)), 3)}
     else:
         roofline = {
-            "kernel": "pm_ns_gemm_kernel",
+            # a lone mid-size matrix (config 1) runs every stage on the small-tile engine
+            "kernel": "pm_ns_gemm_kernel" if any(r["tile"] == 256 for r in gemm) else "pm_tile_gemm_kernel",
             "bound": "mfma",
             "achieved": round(achieved, 2),
             "peak": PEAK_BF16_TFLOPS,

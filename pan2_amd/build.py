@@ -6,8 +6,8 @@ extension _pm_host with g++ against torch's headers.
 The library is plain C ABI (include/panmuon.h) and links the HIP runtime by
 SONAME (libamdhip64.so.7), so inside a process that already imported torch it
 binds to torch's runtime; /opt/rocm/lib is the rpath fallback when loaded alone.
-_pm_host (csrc/pm_host.cpp) has no device code: it fills pm_adam_tensor
-descriptors from torch's tensor lists for the AdamW path.
+_pm_host (csrc/pm_host.cpp) has no device code: it fills pm_adam_tensor and
+pm_matrix descriptors from torch's tensor lists (the AdamW and the Muon step).
 """
 from __future__ import annotations
 

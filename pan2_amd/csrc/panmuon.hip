@@ -699,8 +699,14 @@ struct StageEngine {
 // time in us. An item's time at a tile edge is an overhead plus its units of
 // 64 k; the coefficients are fits to per-launch times (rocprof) of lone and
 // grouped matrices from 256 x 256 to 5120 x 5120 and 4096 x 12288, measured at
-// all three edges, within some 15%. Bits do not depend on
-// the choice (the accumulation order of an element is the same at any edge).
+// all three edges, on the MI355X's 256 CUs. Most launches come within 15% of
+// their estimate. The products of several matrices run longer, at every edge
+// alike: 15 of a width-1024 block take 52 us on 256-tiles and 40 on 128, with
+// estimates of 39 and 30, three of 777 x 1900 take 35 and 9.7 (64) with 29 and
+// 7.2; the block's grams take 64 on 128 with 52. At 4 x 5120 x 5120 the 128
+// estimate is 19% high (663 for 558). In these the faster edge is still the one
+// chosen. Bits do not depend on the choice (the accumulation order of an element
+// is the same at any edge).
 //   256: one round of n <= 256 items 17 + (0.85 + 0.85 n/256)·units, more
 //        rounds 11 + 1.4·units each (lone 1024 x 1024 product 30 us at 10
 //        items, 4096 x 4096 128 us at 256);

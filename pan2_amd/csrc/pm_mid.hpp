@@ -13,9 +13,9 @@
 // side has); what lies beyond stays unwritten and is never multiplied in.
 //
 // Measured (per launch, GRAM / SYMM / UPDATE, us, 256-tile engine -> here):
-// lone 1024 x 4096 30+9 / 30 / 36 -> 14+5 / 7.5 / 15 (K-split GRAM + reduce);
-// 256 x 1000 23 / 15 / 17 -> 6.8 / 5.1 / 4.9; 14 matrices of a width-1024
-// block 124 / 47 / 99 -> 60 / 38 / 99 (UPDATE stays on 256). At 4 of 5120 x
+// lone 1024 x 4096 29+9 / 30 / 36 -> 14+5 / 7.8 / 14 (K-split GRAM + reduce);
+// 256 x 1000 23 / 15 / 17 -> 7.0 / 5.2 / 5.0; the 15 matrices of a width-1024
+// block 142 / 52 / 100 -> 64 / 40 / 100 (UPDATE stays on 256). At 4 of 5120 x
 // 5120 the 128 tile runs 558 / 573 / 1084 against 457 / 470 / 810: its
 // operands cross the L2 twice as often, so large stages keep 256.
 //
